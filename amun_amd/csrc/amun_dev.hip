@@ -49,7 +49,7 @@ struct amun_ctx {
   // launch shapes of the sweeps (workgroup size, XCD-aware order), per
   // direction; set by amun_dev_autotune
   int wg[3] = {256, 256, 256};
-  int swz[3] = {0, 0, 0};
+  int swz[3] = {1, 1, 1};
   // captured steps: one graph per (cmax slot, primitive buffer, dtnext)
   bool use_graph = false;
   struct Graph { int slot, qcur; double dtnext; hipGraphExec_t exec; };
@@ -381,14 +381,28 @@ int validate_grid(const amun_cfg& c, const amun_grid& g) {
   return 0;
 }
 
-// LDS bytes of the sweep along dir (chunked pencil I/O of the x and y
-// sweeps: primitive slots, increment slots, kLdsLanes lanes each)
-size_t sweep_lds(const amun_ctx* c, int dir, int /*wg*/) {
-  const bool chunk = dir < 2, last = dir == c->rc.nd - 1;
-  const bool chunk_d = c->qsize == 8;   // sweep_chunk_d<T>()
-  const bool din = chunk && dir > 0 && chunk_d, dout = chunk && !last && chunk_d;
-  const int nbuf = (chunk ? 1 : 0) + ((din || dout) ? 1 : 0);
-  return (size_t)nbuf * 4 * c->nv * kLdsLanes * c->qsize;
+// launch shape of a sweep along dir: np pencils of nc + 2 lanes each per
+// workgroup, the lanes, the workgroups and the LDS.  Of the even np with at
+// most wg lanes (at least two pencils), the one that leaves the fewest lanes
+// idle: 14 pencils on 252 of 256 lanes at nc = 16.
+struct SweepShape {
+  int np, lanes;
+  unsigned grid;
+  size_t lds;
+};
+
+SweepShape sweep_shape(const amun_ctx* c, int dir, int wg) {
+  const RunConst& rc = c->rc;
+  const long long total = (long long)rc.nblk * (rc.nd == 3 ? rc.nc * rc.nc : rc.nc);
+  const auto lanes = [&](int np) { return (np * (rc.nc + 2) + 63) / 64 * 64; };
+  SweepShape s;
+  s.np = 2;
+  for (int np = 2; lanes(np) <= wg; np += 2)
+    if ((long long)np * lanes(s.np) >= (long long)s.np * lanes(np)) s.np = np;
+  s.lanes = lanes(s.np);
+  s.grid = (unsigned)((total + s.np - 1) / s.np);
+  s.lds = sweep_lds_elems(c->nv, c->disp.R, rc.nc, s.np, dir) * c->qsize;
+  return s;
 }
 
 // the slopes of the multi-dimensional limiting of the stage input Q[qcur]
@@ -616,7 +630,8 @@ static int init_device(amun_ctx* c, const std::vector<int32_t>& nbr,
   ALLOC(c->scratch, (size_t)std::max(4096 * 8, 2 * nruns) * sizeof(double));
   {
     const long long npen = nd == 3 ? (long long)rc.nc * rc.nc : rc.nc;
-    c->nspart = (int)((rc.nblk * npen + 63) / 64);
+    // at least two pencils per workgroup, see sweep_shape
+    c->nspart = (int)((rc.nblk * npen + 1) / 2);
     ALLOC(c->spart, (size_t)c->nspart * sizeof(SpeedPart));
   }
   if (cfg->mlp_limiting) {
@@ -682,11 +697,10 @@ static int init_device(amun_ctx* c, const std::vector<int32_t>& nbr,
     amun_dev_finalize(c);
     return fail(600, "no kernel instantiation for this configuration");
   }
-  // the x and y sweeps stage pencil chunks in LDS: allow the largest
-  // workgroup's share (above the 64 KiB default of dynamic LDS)
+  // allow the sweeps' LDS (above the 64 KiB default of dynamic LDS)
   for (int dir = 0; dir < nd; dir++) {
-    const size_t lds = sweep_lds(c, dir, 256);
-    if (!lds) continue;
+    size_t lds = 0;
+    for (int wg : {64, 128, 256}) lds = std::max(lds, sweep_shape(c, dir, wg).lds);
     e = hipFuncSetAttribute((const void*)c->disp.sweep[dir],
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) {
@@ -1436,13 +1450,11 @@ static int enqueue_step(amun_ctx* c, double dtnext, int slot, int qcur, hipEvent
                         double* rec = nullptr) {
   Dispatch& d = dispatch_of(c);
   const RunConst& rc = c->rc;
-  const int npen = (rc.nd == 3) ? rc.nc * rc.nc : rc.nc;
-  const long long nthreads = (long long)rc.nblk * npen;
-
   const std::vector<StageDef> stages = stage_table(c);
   if (rec)   // stage inputs: U^n, then every intermediate stage output
     HIP_TRY(hipMemcpyAsync(rec, c->U0, c->nstate * sizeof(double), hipMemcpyDeviceToDevice,
                            c->stream));
+  int parts = 0;   // workgroups of the last sweep
   for (size_t s = 0; s < stages.size(); s++) {
     if (c->amr.on) {
       int r = amr_fill(c, qcur, slot);
@@ -1500,20 +1512,7 @@ static int enqueue_step(amun_ctx* c, double dtnext, int slot, int qcur, hipEvent
     a.ca = stages[s].ca;
     a.cb = stages[s].cb;
     a.dtnext = dtnext;
-    if (c->fuse) {
-      // every workgroup of 256 lanes holds whole blocks in each direction
-      a.first = (s == 0);
-      a.swz = c->swz[0];
-      const dim3 grid((unsigned)((nthreads + 255) / 256)), block(256);
-      const size_t lds = std::max(sweep_lds(c, 0, 256), sweep_lds(c, 1, 256));
-      hipLaunchKernelGGL(d.stage, grid, block, lds, c->stream, a, rc);
-      if (a.last)
-        hipLaunchKernelGGL(k_reduce_speed, dim3(1), dim3(1024), 0, c->stream, c->spart,
-                           (int)grid.x, c->rs, slot ^ 1, rc.nruns);
-      if (ev) HIP_TRY(hipEventRecord(*ev++, c->stream));
-    }
-    for (int dir = 0; dir < rc.nd && !c->fuse; dir++) {
-      const int wg = c->wg[dir];
+    for (int dir = 0; dir < rc.nd; dir++) {
       a.first = (s == 0 && dir == 0);
       if (d.compact[dir]) {
         const long long nt = (long long)rc.nblk * (rc.nd == 3 ? rc.nc * rc.nc : rc.nc) * c->nv;
@@ -1522,20 +1521,21 @@ static int enqueue_step(amun_ctx* c, double dtnext, int slot, int qcur, hipEvent
                            c->st);
       }
       a.swz = c->swz[dir];
-      const dim3 grid((unsigned)((nthreads + wg - 1) / wg)), block(wg);
-      hipLaunchKernelGGL(d.sweep[dir], grid, block, sweep_lds(c, dir, wg), c->stream, a, rc);
-      if (a.last && dir == rc.nd - 1)
-        hipLaunchKernelGGL(k_reduce_speed, dim3(1), dim3(1024), 0, c->stream, c->spart,
-                           (int)grid.x, c->rs, slot ^ 1, rc.nruns);
-      if (ev) HIP_TRY(hipEventRecord(*ev++, c->stream));
+      const SweepShape w = sweep_shape(c, dir, c->wg[dir]);
+      a.np = w.np;
+      hipLaunchKernelGGL(d.sweep[dir], dim3(w.grid), dim3(w.lanes), w.lds, c->stream, a, rc);
+      parts = (int)w.grid;
+      if (ev && !c->fuse) HIP_TRY(hipEventRecord(*ev++, c->stream));
     }
+    if (ev && c->fuse) HIP_TRY(hipEventRecord(*ev++, c->stream));
     qcur ^= 1;
     if (rec && s + 1 < stages.size())
       HIP_TRY(hipMemcpyAsync(rec + (s + 1) * c->nstate, stages[s].to_u0 ? c->U0 : c->U1,
                              c->nstate * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
   }
-  hipLaunchKernelGGL(k_end_step, dim3((unsigned)((rc.nruns + 255) / 256)), dim3(256), 0,
-                     c->stream, c->rs, c->trace, c->tsteps, rc, slot, dtnext);
+  hipLaunchKernelGGL(k_end_step, dim3((unsigned)std::max(1, std::min(64, parts / 1024))),
+                     dim3(64 * kEndWaves), 0, c->stream, c->spart, parts, c->rs, c->trace,
+                     c->tsteps, rc, slot, dtnext);
   if (ev) HIP_TRY(hipEventRecord(*ev++, c->stream));
   HIP_TRY(hipGetLastError());
   return 0;
@@ -1755,16 +1755,15 @@ int amun_dev_autotune(amun_ctx* c, int32_t nsteps, int32_t* choice) {
   c->use_graph = false;
   const int wgs[3] = {64, 128, 256};
   double best[3] = {1e300, 1e300, 1e300};
-  int bwg[3] = {256, 256, 256}, bsw[3] = {0, 0, 0};
+  int bwg[3] = {256, 256, 256}, bsw[3] = {1, 1, 1};
   const int nk = kernels_per_step(c);
   std::vector<double> kms(nk);
   int r = 0;
-  // the chunked x and y sweeps stage kLdsLanes lanes of LDS per workgroup
-  // whatever its size, so only full workgroups fill a CU there
+  // the x and y sweeps keep workgroups of kSweepLanes lanes
   for (int w = 0; w < 3 && !r; w++)
     for (int z = 0; z < 2 && !r; z++) {
       for (int dir = 0; dir < nd; dir++) {
-        c->wg[dir] = dir < 2 ? kLdsLanes : wgs[w];
+        c->wg[dir] = dir < 2 ? kSweepLanes : wgs[w];
         c->swz[dir] = z;
       }
       double ms = 0.0;
@@ -1797,7 +1796,7 @@ int amun_dev_set_launch(amun_ctx* c, const int32_t* choice) {
   for (int dir = 0; dir < c->rc.nd; dir++) {
     const int wg = choice[2 * dir];
     if (wg != 64 && wg != 128 && wg != 256) return fail(500, "workgroup size must be 64, 128 or 256");
-    if (dir < 2 && wg != kLdsLanes)
+    if (dir < 2 && wg != kSweepLanes)
       return fail(500, "the x and y sweeps run workgroups of 256 lanes");
   }
   HIP_TRY(hipStreamSynchronize(c->stream));

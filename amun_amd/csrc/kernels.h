@@ -15,16 +15,17 @@
 // value the reference copies into its ghost layers (boundaries.F90:372-479,
 // same-level face/edge/corner copies).
 //
-// One RK stage = one sweep kernel per direction.  A sweep thread owns one
-// pencil of a block and walks it with a sliding window: each cell is
-// reconstructed once (both faces), each face gets one Riemann solve, and the
-// flux difference goes straight into the cell's increment.  The x sweep
-// stores -dxi*dF, the y sweep subtracts dyi*dF, and the last sweep completes
-// du, applies the stage combine of the integrator, the psi decay, recomputes
-// the primitive variables of the new state and (last stage) reduces the
-// maximum speed for the next CFL step -- i.e. update_fluxes, update_increment,
-// the stage update and update_variables of evolution.F90:1005-2094 fused into
-// nd kernels.  dt, cmax and the simulation time stay on the device.
+// One RK stage = one sweep kernel per direction.  A sweep lane owns one cell
+// of a pencil: it reconstructs the cell once (both faces), solves the Riemann
+// problem of the cell's lower face, and puts the flux difference straight
+// into the cell's increment; the states and fluxes of the neighbouring cells
+// pass through LDS.  The x sweep stores -dxi*dF, the y sweep subtracts
+// dyi*dF, and the last sweep completes du, applies the stage combine of the
+// integrator, the psi decay, recomputes the primitive variables of the new
+// state and (last stage) reduces the maximum speed for the next CFL step --
+// i.e. update_fluxes, update_increment, the stage update and
+// update_variables of evolution.F90:1005-2094 fused into nd kernels.  dt,
+// cmax and the simulation time stay on the device.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -133,11 +134,21 @@ __device__ __forceinline__ double dt_of(const RunConst& rc, const RunState* R,
 // them within four steps.  Requires nc % 4 == 0.
 // FP32 arrays (element size 4) of 3D runs use 4x4x2 bricks instead, so that
 // a line (32 floats) again spans four steps of every sweep direction.
+// All factors are below 2^24, which the masks tell the compiler: the products
+// are the full-rate 24-bit ones (a 32-bit product takes four times as long).
+__host__ __device__ __forceinline__ int mul24(int a, int b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return (int)(((unsigned)a & 0xffffffu) * ((unsigned)b & 0xffffffu));
+#else
+  return a * b;
+#endif
+}
+
 template <int ES>
 __host__ __device__ __forceinline__ int lidx(int nc, int nd, int i, int j, int k) {
-  if (nd == 2) return (((i >> 2) * nc + j) << 2) | (i & 3);
-  if (ES == 8) return ((((i >> 2) * nc + k) * nc + j) << 2) | (i & 3);
-  return (((((i >> 2) * (nc >> 1) + (k >> 1)) * nc + j) * 2 + (k & 1)) << 2) | (i & 3);
+  if (nd == 2) return ((mul24(i >> 2, nc) + j) << 2) | (i & 3);
+  if (ES == 8) return ((mul24(mul24(i >> 2, nc) + k, nc) + j) << 2) | (i & 3);
+  return (((mul24(mul24(i >> 2, nc >> 1) + (k >> 1), nc) + j) * 2 + (k & 1)) << 2) | (i & 3);
 }
 
 // position of (i,j,k), possibly outside the block by at most nc, in the pool
@@ -231,8 +242,8 @@ __device__ __forceinline__ void riemann(const EosConst<T>& e, const SrConst& sc,
   else riemann_hll<P, T>(e, cmax, cmax2, ql, qr, f);
 }
 
-// lanes of the per-lane LDS slots of the chunked (x and y) sweeps
-constexpr int kLdsLanes = 256;
+// lanes of the x and y sweeps' workgroups
+constexpr int kSweepLanes = 256;
 
 // maximum speed of one sweep workgroup for the next CFL step, and its run
 // (run < 0: the workgroup spanned several runs and used atomics instead)
@@ -256,6 +267,7 @@ struct SweepArgs {
   SpeedPart* spart;                // per-workgroup maximum speeds (last stage)
   int slot;                        // cmax slot of this step
   int swz;                         // XCD-aware workgroup order (autotuned)
+  int np;                          // pencils per workgroup
   int kind;                        // stage combine, see combine()
   int last;                        // last stage of the step
   int comp;                        // the stage writes the step state U0
@@ -940,7 +952,7 @@ __device__ __forceinline__ void wave_max_speed(RunState* rs, int run, int slot, 
 }
 
 // Maximum speed of a sweep workgroup (at most kMaxWaves waves) into
-// part[blockIdx.x], reduced over the workgroups by k_reduce_speed after the
+// part[blockIdx.x], reduced over the workgroups by k_end_step after the
 // sweep.  Device-scope atomics on one address from every wave of a 256^3
 // sweep (16K of them) serialise at the memory side; a workgroup whose lanes
 // belong to more than one run (a batch) still uses them.  Every thread of
@@ -984,420 +996,459 @@ __device__ __forceinline__ void wg_max_speed(RunState* rs, SpeedPart* part, int 
   }
 }
 
-// The per-workgroup maxima of the last sweep into the runs' cmax slots (one
-// workgroup of 1024 threads; per-run maxima in LDS when the runs fit)
-constexpr int kReduceRuns = 2048;
-static __global__ __launch_bounds__(1024) void k_reduce_speed(const SpeedPart* __restrict__ part,
-                                                              int n, RunState* rs, int slot,
-                                                              int nruns) {
-  __shared__ unsigned long long lm[kReduceRuns];
-  if (nruns <= kReduceRuns) {
-    for (int r = threadIdx.x; r < nruns; r += blockDim.x) lm[r] = 0ull;
-    __syncthreads();
-    if (nruns == 1) {
-      double m = 0.0;
-      for (int i = threadIdx.x; i < n; i += blockDim.x)
-        if (part[i].run == 0) m = fmax(m, part[i].smax);
-      for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off));
-      if ((threadIdx.x & 63) == 0 && m > 0.0)
-        atomicMax(&lm[0], (unsigned long long)__double_as_longlong(m));
-    } else {
-      for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        const SpeedPart p = part[i];
-        if (p.run >= 0 && p.smax > 0.0)
-          atomicMax(&lm[p.run], (unsigned long long)__double_as_longlong(p.smax));
+// The end of a step: the per-workgroup maxima of its last sweep into the runs'
+// cmax slots for the next step, and (first workgroup) each run's dt into the
+// trace ring trace[(step mod tsteps) * nruns + run], its time and its step
+// advanced.  A wave takes a contiguous range of the maxima, which mostly
+// belong to one run, and sends one atomic per run it met: with one workgroup
+// and an LDS atomic per entry, the 30 K entries of a 16-run batch took 1.1 ms.
+constexpr int kEndWaves = 4;
+static __global__ __launch_bounds__(64 * kEndWaves) void k_end_step(
+    const SpeedPart* __restrict__ part, int n, RunState* rs, double* trace, int tsteps,
+    RunConst rc, int slot, double dtnext) {
+  const int lane = threadIdx.x & 63, w = blockIdx.x * kEndWaves + (threadIdx.x >> 6);
+  const int per = ((n + (int)gridDim.x * kEndWaves - 1) / ((int)gridDim.x * kEndWaves) + 63) & ~63;
+  double acc = 0.0;
+  int cur = -1;
+  auto flush = [&]() {
+    double m = acc;
+    for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off));
+    if (lane == 0 && cur >= 0 && m > 0.0)
+      atomicMax(&rs[cur].cmax_bits[slot ^ 1], (unsigned long long)__double_as_longlong(m));
+    acc = 0.0;
+  };
+  for (int i0 = w * per; i0 < n && i0 < (w + 1) * per; i0 += 64) {
+    SpeedPart p = {0.0, -1, 0};
+    if (i0 + lane < n) p = part[i0 + lane];
+    const int r0 = __shfl(p.run, 0);
+    if (__all(p.run == r0 || i0 + lane >= n)) {
+      if (r0 != cur) {
+        flush();
+        cur = r0;
       }
+      acc = fmax(acc, p.smax);
+    } else if (p.run >= 0 && p.smax > 0.0) {
+      atomicMax(&rs[p.run].cmax_bits[slot ^ 1], (unsigned long long)__double_as_longlong(p.smax));
     }
-    __syncthreads();
-    for (int r = threadIdx.x; r < nruns; r += blockDim.x)
-      if (lm[r]) atomicMax(&rs[r].cmax_bits[slot], lm[r]);
-  } else {
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-      const SpeedPart p = part[i];
-      if (p.run >= 0 && p.smax > 0.0)
-        atomicMax(&rs[p.run].cmax_bits[slot], (unsigned long long)__double_as_longlong(p.smax));
+  }
+  flush();
+  if (blockIdx.x == 0) {
+    for (int r = threadIdx.x; r < rc.nruns; r += blockDim.x) {
+      RunState* R = rs + r;
+      const double dt = dt_of(rc, R, slot, dtnext);
+      trace[(size_t)(R->step % tsteps) * rc.nruns + r] = dt;
+      R->dt = dt;
+      R->time += dt;
+      R->step += 1;
     }
   }
 }
 
-// ---------------------------------------------------------------------------
-// the sweep kernel
-// ---------------------------------------------------------------------------
-// FP64 sweeps hold more than 256 registers per lane and run one wave per
-// SIMD (spilling to reach two is several times slower); FP32 sweeps fit two.
-template <typename T>
-constexpr int sweep_min_waves() { return sizeof(T) == 4 ? 2 : 1; }
+// new_time_step: cmax = tiny before the reduction of the next step, one
+// thread per run (first sweep of a step)
+__device__ __forceinline__ void reset_speed(const SweepArgs& a, const RunConst& rc) {
+  if (!a.first) return;
+  for (long long r = (long long)blockIdx.x * blockDim.x + threadIdx.x; r < rc.nruns;
+       r += (long long)gridDim.x * blockDim.x)
+    a.rs[r].cmax_bits[a.slot ^ 1] = (unsigned long long)__double_as_longlong(kTiny);
+}
 
-// The FP64 x and y sweeps also move the increment through LDS in chunks; the
-// FP32 ones read and write it per cell, which leaves LDS for two workgroups
-// per CU.
+// ---------------------------------------------------------------------------
+// the sweep kernels
+// ---------------------------------------------------------------------------
 #include "mlp.h"
 
-template <typename T>
-constexpr bool sweep_chunk_d() { return sizeof(T) == 8; }
+// Waves per SIMD the sweeps are compiled for.  One lane works on one cell, so
+// that besides the HLLD temporaries (118 registers in FP64) nothing has to
+// stay in registers over a solve: four waves per SIMD (128 registers) hide
+// the FP64 latencies.  The relativistic solvers (quartic, root search) and
+// the Roe eigensystem need more registers.
+template <class P, int RS, typename T>
+constexpr int sweep_min_waves() {
+  if (P::sr) return P::mhd ? 2 : 3;
+  return RS == RS_ROE && P::mhd && sizeof(T) == 8 ? 2 : 4;
+}
 
-// the sweep along DIR of one workgroup: its lanes walk the pencils
-// workgroup_index(swz) * blockDim.x + threadIdx.x along DIR.  Every thread
-// of the workgroup must call it (the last sweep reduces the maximum speed
-// over the workgroup).
+// Lanes of a sweep workgroup: the interior cells of its np pencils, then the
+// cells before and behind each pencil.
+// LDS, in elements of T: the pencils' primitive state with R + 1 cells beyond
+// each end, then in its place the upper face states, then the fluxes.  The
+// width of a pencil's row is the smallest that spreads the lanes of a wave
+// over all banks: four cells by four pencils (x), four pencils by sixteen
+// cells (y), one cell each (z).
+__host__ __device__ constexpr int row_width(int n, int dir) {
+  return dir == 0 ? (n + 3) / 8 * 8 + 4 : (dir == 1 ? (n + 7) / 16 * 16 + 8 : n | 1);
+}
+__host__ __device__ constexpr int tile_width(int nc, int R, int dir) {
+  return row_width(nc + 2 * (R + 1), dir);
+}
+__host__ __device__ constexpr int face_width(int nc, int dir) { return row_width(nc + 1, dir); }
+__host__ __device__ constexpr size_t sweep_lds_elems(int nv, int R, int nc, int np, int dir) {
+  const int w = R ? tile_width(nc, R, dir) : face_width(nc, dir);
+  return (size_t)nv * np * w;
+}
+
+// n / d for 0 <= n < 2^16, d > 0, with rd = 1 / d (exact: the distance of
+// (n + 0.5) / d from an integer is at least 0.5 / d)
+__device__ __forceinline__ int quot(int n, float rd) { return (int)((float(n) + 0.5f) * rd); }
+
+// x[o / sizeof(X)] with a 32-bit byte offset o on a base that is the same in
+// the whole wave: the base stays in scalar registers, and an access to
+// another variable costs no vector address arithmetic
+template <typename X>
+__device__ __forceinline__ X& at_byte(X* x, unsigned o) {
+  using B = std::conditional_t<std::is_const<X>::value, const char, char>;
+  return *reinterpret_cast<X*>(reinterpret_cast<B*>(x) + o);
+}
+
+// The sweep along DIR of the pencils g0 .. g0 + np - 1 of the pool (np
+// even), one lane per cell.  The cells are
+// staged in LDS; each lane reconstructs its cell, leaves its upper face state
+// in LDS, solves the Riemann problem of its lower face with the state of the
+// cell before it, leaves the flux in LDS and updates its cell with the flux of
+// the cell behind it.  The interior lanes go over the cells in the order of
+// the 4-cell bricks, so that every access of a wave to its own cells is whole
+// 128-byte lines: with a pencil's cells on consecutive lanes instead, the z
+// sweep of the 128^3 MHD run sent 14.2 M write requests to L2 for 4.7 M full
+// ones and took 2.4 ms at 256^3.  Every thread of the workgroup must call
+// this.  Returns the maximum speed of the lane's new state (last sweep of a
+// step).
 template <class P, int REC, int RS, int ND, int DIR, typename T>
-__device__ __forceinline__ void sweep_body(const SweepArgs& a, const RunConst& rc) {
+__device__ __forceinline__ double sweep_cells(const SweepArgs& a, const RunConst& rc, int g0,
+                                              int np, T* smem, int& run) {
   constexpr int NV = P::nv;
-  constexpr bool kLast = (DIR == ND - 1);
+  constexpr bool kLast = DIR == ND - 1;
+  constexpr bool kPair = sizeof(T) == 4 && ND == 3;   // bricks of two z planes (lidx)
   using RC = Recon<P, REC, ND, DIR, T>;
-  // chunked pencil I/O along x and y (see loadq below)
-  constexpr bool kChunk = DIR < 2;
-  constexpr bool kDin = kChunk && DIR > 0 && sweep_chunk_d<T>();    // increment read in chunks
-  constexpr bool kDout = kChunk && !kLast && sweep_chunk_d<T>();    // increment written in chunks
-  // per-lane LDS slots of the chunked pencil I/O: sq holds four cells of the
-  // primitive window, sd four cells of the increment (4 NV values per lane
-  // each), slot-major with a fixed stride of kLdsLanes lanes (consecutive
-  // lanes hit consecutive banks; a compile-time stride keeps the slot
-  // addresses out of the register file).  The chunked sweeps launch
-  // workgroups of at most kLdsLanes lanes.
-  extern __shared__ __align__(16) unsigned char smem[];
-  constexpr int wg = kLdsLanes;
-  T* const sq = reinterpret_cast<T*>(smem);
-  T* const sd = sq + (kChunk ? 4 * NV * wg : 0);
-  const int nc = rc.nc;
-  const int npen = (ND == 3) ? nc * nc : nc;
-  const long long gid = (long long)workgroup_index(a.swz) * blockDim.x + threadIdx.x;
-  const int b = (int)(gid / npen);
-  const int t = (int)(gid % npen);
-  const bool active = b < rc.nblk;
+  constexpr int R = RC::R;
+  const int nc = rc.nc, npen = (ND == 3) ? nc * nc : nc;
+  const int wt = tile_width(nc, R, DIR), wf = face_width(nc, DIR), nf = np * wf;
+  T* const face = smem;   // [var][pencil][cell + 1] upper states, [var][pencil][cell] fluxes
+  const int b0 = g0 / npen, t0 = g0 - b0 * npen;
+  const float rnpen = 1.0f / float(npen), rnc = 1.0f / float(nc), rnp = 1.0f / float(np);
 
-  if (a.first && gid < rc.nruns) {
-    // reset the maximum-speed accumulators of the next step (new_time_step:
-    // cmax = tiny before the reduction), one thread per run
-    a.rs[gid].cmax_bits[a.slot ^ 1] = (unsigned long long)__double_as_longlong(kTiny);
+  // block, transverse coordinates of local pencil q
+  auto pencil = [&](int q, int& b, int& c1, int& c2) {
+    int t = t0 + q;
+    const int db = quot(t, rnpen);
+    b = b0 + db;
+    t -= db * npen;
+    if constexpr (ND == 2) {
+      c1 = t;
+      c2 = 0;
+    } else if constexpr (DIR == 2) {
+      const int h = quot(t >> 2, rnc);            // (i & 3) + 4 (j + nc (i >> 2))
+      c1 = (h << 2) | (t & 3);
+      c2 = (t >> 2) - h * nc;
+    } else if constexpr (!kPair) {
+      c2 = quot(t, rnc);                          // j + nc k, i + nc k
+      c1 = t - c2 * nc;
+    } else if constexpr (DIR == 0) {
+      const int h = quot(t >> 1, rnc);            // (k & 1) + 2 (j + nc (k >> 1))
+      c1 = (t >> 1) - h * nc;
+      c2 = (h << 1) | (t & 1);
+    } else {                                      // (i & 3) + 4 (k & 1) + 8 (i / 4 + nc / 4 (k / 2))
+      const int h = quot(t >> 3, 4.0f * rnc), m = (t >> 3) - h * (nc >> 2);
+      c1 = (m << 2) | (t & 3);
+      c2 = (h << 1) | ((t >> 2) & 1);
+    }
+  };
+  auto coords = [&](int cc, int c1, int c2, int& i, int& j, int& k) {
+    if constexpr (DIR == 0) { i = cc; j = c1; k = c2; }
+    else if constexpr (DIR == 1) { i = c1; j = cc; k = c2; }
+    else { i = c1; j = c2; k = cc; }
+  };
+
+  // the lane's pencil p and cell c
+  const int lane = threadIdx.x, nin = np * nc;
+  int p, c;
+  if (lane < nin) {
+    if constexpr (DIR == 0) {
+      const int h = quot(lane >> 2, rnp);
+      p = (lane >> 2) - h * np;
+      c = (h << 2) | (lane & 3);
+    } else if constexpr (DIR == 1) {
+      constexpr int G = kPair ? 3 : 2;            // pencils side by side in a brick line
+      const int h = quot(lane >> G, rnc);
+      p = (h << G) | (lane & ((1 << G) - 1));
+      c = (lane >> G) - h * nc;
+      if (p >= (np >> G << G)) {                  // the last, incomplete line: two by two
+        const int r = lane - (np >> G << G) * nc, g = quot(r >> 1, rnc);
+        p = (np >> G << G) + 2 * g + (r & 1);
+        c = (r >> 1) - g * nc;
+      }
+    } else if constexpr (kPair) {
+      const int h = quot(lane >> 1, rnp), r = lane - 2 * h * np, m = np & ~3;
+      p = ((r >> 3) << 2) | (r & 3);
+      c = (h << 1) | ((r >> 2) & 1);
+      if (r >= 2 * m) {                           // the last two pencils
+        p = m + (r & 1);
+        c = (h << 1) | ((r >> 1) & 1);
+      }
+    } else {
+      c = quot(lane, rnp);
+      p = lane - c * np;
+    }
+  } else {
+    p = lane - nin;
+    c = -1;
+    if (p >= np) { p -= np; c = nc; }
+  }
+  int b, c1, c2, ci, cj, ck;
+  pencil(p < np ? p : 0, b, c1, c2);
+  coords(c, c1, c2, ci, cj, ck);
+  const bool active = p < np && b < rc.nblk, inner = active && lane < nin;
+  const T* __restrict__ Qp = static_cast<const T*>(a.Q);
+  // the lane's own cell, relative to the workgroup's first block: 32-bit
+  // offsets on uniform bases
+  const size_t nbk = (size_t)NV * rc.ncell;
+  const unsigned ob = inner ? (unsigned)(b - b0) * (unsigned)nbk : 0u;
+  const unsigned ot = inner ? ob + lidx<sizeof(T)>(nc, ND, ci, cj, ck) : 0u;
+  const size_t base0 = (size_t)b0 * nbk;
+
+  if constexpr (R > 0) {
+    if (inner) {
+      const T* __restrict__ Q0 = Qp + base0;
+#pragma unroll
+      for (int v = 0; v < NV; v++) smem[(v * np + p) * wt + c + R + 1] = at_byte(Q0 + v * rc.ncell, ot * (unsigned)sizeof(T));
+    }
+    // the R + 1 cells beyond each end
+    constexpr int H = 2 * (R + 1);
+    for (int x = lane; x < np * H; x += blockDim.x) {
+      const int ph = x / H, m = x - ph * H, ch = m <= R ? m - 1 - R : nc + m - 1 - R;
+      int hb, h1, h2, i, j, k;
+      pencil(ph, hb, h1, h2);
+      if (hb < rc.nblk) {
+        coords(ch, h1, h2, i, j, k);
+        const size_t pk = cell_index<sizeof(T)>(a.nbr, rc, hb, i, j, k);
+        const T* __restrict__ Qh = Qp + ((pk >> 32) * nbk + (pk & 0xffffffffull));
+#pragma unroll
+        for (int v = 0; v < NV; v++) smem[(v * np + ph) * wt + ch + R + 1] = Qh[v * rc.ncell];
+      }
+    }
+    __syncthreads();
   }
 
-  const int run = active ? a.brun[b] : 0;
-  const RunState* R = a.rs + run;
-  const double cmaxd = cmax_of(R, a.slot);
+  run = a.brun[b < rc.nblk ? b : b0];   // lanes without a cell: the first block's
+  const RunState* Rs = a.rs + run;
+  const double cmaxd = cmax_of(Rs, a.slot);
   const T cmax = T(cmaxd), cmax2 = T(cmaxd * cmaxd);
-  const double dt = dt_of(rc, R, a.slot, a.dtnext);
-  const double ds = a.fac * dt;
   const EosConst<T> e{T(rc.gamma), T(rc.gammam1), T(rc.gammam1i), T(rc.csnd), T(rc.csnd2)};
-  const EosConst<double> ed{rc.gamma, rc.gammam1, rc.gammam1i, rc.csnd, rc.csnd2};
-  const T* __restrict__ Qp = static_cast<const T*>(a.Q);
-  T* __restrict__ Dp = static_cast<T*>(a.D);
-  T* __restrict__ Qo = static_cast<T*>(a.Qout);
   double smax = 0.0;
 
+  T flc[NV], frc[NV], f[NV];
   if (active) {
-    // transverse coordinates of the pencil
-    int c1 = t % nc, c2 = (ND == 3) ? t / nc : 0;
-    auto coords = [&](int c, int& i, int& j, int& k) {
-      if constexpr (DIR == 0) { i = c; j = c1; k = c2; }
-      else if constexpr (DIR == 1) { i = c1; j = c; k = c2; }
-      else { i = c1; j = c2; k = c; }
-    };
-    // x and y sweeps move their pencil data in chunks of four cells: a
-    // brick line spans four cells along x and along y, so loading (and
-    // storing) four cells at once uses whole lines instead of a quarter of a
-    // line per walk step.  The chunks live in per-lane LDS slots.
-    const int tid = threadIdx.x;
-    auto loadq = [&](int c, T* q) {
-      if constexpr (kChunk) {
-        const int first = -1 - RC::R;
-        if (c == first || (c & 3) == 0) {
-          const int c0 = c & ~3;
-#pragma unroll
-          for (int m = 0; m < 4; m++) {
-            int i, j, k;
-            coords(c0 + m, i, j, k);
-            const size_t pk = cell_index<sizeof(T)>(a.nbr, rc, b, i, j, k);
-#pragma unroll
-            for (int v = 0; v < NV; v++) sq[(m * NV + v) * wg + tid] = Qp[var_index<NV>(rc, pk, v)];
-          }
-        }
-#pragma unroll
-        for (int v = 0; v < NV; v++) q[v] = sq[((c & 3) * NV + v) * wg + tid];
-      } else {
-        int i, j, k;
-        coords(c, i, j, k);
-        size_t pk = cell_index<sizeof(T)>(a.nbr, rc, b, i, j, k);
-#pragma unroll
-        for (int v = 0; v < NV; v++) q[v] = Qp[var_index<NV>(rc, pk, v)];
-      }
-    };
-    // global offsets (without the variable term) of the four cells of the
-    // increment chunk that starts at cell c0
-    auto dchunk_base = [&](int c0, size_t* base) {
-#pragma unroll
-      for (int m = 0; m < 4; m++) {
-        int i, j, k;
-        coords(c0 + m, i, j, k);
-        base[m] = (size_t)b * NV * (size_t)rc.ncell + (size_t)lidx<sizeof(T)>(nc, ND, i, j, k);
-      }
-    };
-
     // cell size along DIR at this block's level (coordinates.F90:330-341)
-    const double hdir = a.blev ? R->h[DIR] / double(1 << a.blev[b]) : R->h[DIR];
+    const double hdir = a.blev ? Rs->h[DIR] / double(1 << a.blev[b]) : Rs->h[DIR];
     RC rec;
-    T qtmp[NV];
-    // prime the window for cell c = -1: cells -1-R .. -1+R-1
+    if constexpr (R > 0) {
 #pragma unroll
-    for (int m = 0; m < 2 * RC::R; m++) {
-      loadq(-1 - RC::R + m, qtmp);
-      rec.load(m, qtmp);
+      for (int v = 0; v < NV; v++)
+#pragma unroll
+        for (int m = 0; m <= 2 * R; m++) rec.w[v][m] = smem[(v * np + p) * wt + c + 1 + m];
     }
-    T flp[NV], fprev[NV];
-    // unchunked sweeps: the window's next cell is requested one iteration
-    // ahead of its use
-    T qnext[NV];
-    if constexpr (!kChunk) loadq(RC::R - 1, qnext);
-    for (int c = -1; c <= nc; c++) {
-      // operands of the cell finished in this iteration (c-1), loaded before
-      // the reconstruction and Riemann solve so that their latency overlaps
-      // the arithmetic
-      T dpre[NV];
-      double u0pre[NV], u1pre[NV];
-      float cpre[NV];
-      if (c >= 1) {
-        int i, j, k;
-        coords(c - 1, i, j, k);
-        const size_t bb = (size_t)b * NV * (size_t)rc.ncell;
-        const size_t bt = bb + (size_t)lidx<sizeof(T)>(nc, ND, i, j, k);
-        const size_t bd = bb + (size_t)lidx<8>(nc, ND, i, j, k);
-        const size_t bf = bb + (size_t)lidx<4>(nc, ND, i, j, k);
-        if constexpr (kDin) {
-          if (((c - 1) & 3) == 0) {
-            size_t base[4];
-            dchunk_base(c - 1, base);
-#pragma unroll
-            for (int m = 0; m < 4; m++)
-#pragma unroll
-              for (int v = 0; v < NV; v++)
-                sd[(m * NV + v) * wg + tid] = Dp[base[m] + (size_t)v * rc.ncell];
-          }
-        }
-#pragma unroll
-        for (int v = 0; v < NV; v++) {
-          const size_t off = (size_t)v * rc.ncell;
-          if constexpr (DIR > 0 && !kDin) dpre[v] = Dp[bt + off];
-          if constexpr (kLast) {
-            u0pre[v] = a.U0[bd + off];
-            if (a.kind != 0) u1pre[v] = a.U1[bd + off];
-            // the compensation enters the updates of the step state; the
-            // transient stages ignore it (it is below the FP64 rounding of U0)
-            if constexpr (sizeof(T) == 4) cpre[v] = a.comp ? a.C[bf + off] : 0.0f;
-          }
-        }
+    rec.cell(rc, flc, frc, Qp, a.nbr, b, ci, cj, ck, a.st, hdir);
+    if (a.mlps)
+      mlp_apply<P, ND, DIR, T>(rc, Qp, static_cast<const T*>(a.mlps),
+                               static_cast<const T*>(a.mlpg), a.nbr, b, c, c1 + nc * c2, ci, cj,
+                               ck, c == -1 && rc.ng == 2, flc, frc);
+    if constexpr (P::sr) {
+      if (rc.v4) {
+        states_from_4vec<P, T>(flc);
+        states_from_4vec<P, T>(frc);
       }
-      if (c > -1) rec.shift();
-      if constexpr (kChunk) {
-        loadq(c + RC::R, qtmp);
-        rec.load(2 * RC::R, qtmp);
-      } else {
-        rec.load(2 * RC::R, qnext);
-        if (c < nc) loadq(c + RC::R + 1, qnext);
-      }
-      T flc[NV], frc[NV];
-      int ci, cj, ck;
-      coords(c, ci, cj, ck);
-      rec.cell(rc, flc, frc, Qp, a.nbr, b, ci, cj, ck, a.st, hdir);
-      if (a.mlps)
-        mlp_apply<P, ND, DIR, T>(rc, Qp, static_cast<const T*>(a.mlps),
-                                 static_cast<const T*>(a.mlpg), a.nbr, b, c, t, ci, cj, ck,
-                                 c == -1 && rc.ng == 2, flc, frc);
-      if constexpr (P::sr) {
-        if (rc.v4) {
-          states_from_4vec<P, T>(flc);
-          states_from_4vec<P, T>(frc);
-        }
-      }
-      if (c >= 0) {
-        // face c-1/2: left state from cell c-1, right state from cell c
-        T ql[NV], qr[NV], fr[NV], f[NV];
-#pragma unroll
-        for (int p = 0; p < NV; p++) {
-          ql[p] = flp[rot<P, DIR>(p)];
-          qr[p] = frc[rot<P, DIR>(p)];
-        }
-        riemann<P, RS, T>(e, rc.sc, cmax, cmax2, ql, qr, fr);
-#pragma unroll
-        for (int p = 0; p < NV; p++) f[rot<P, DIR>(p)] = fr[p];
-        if (a.ffix && (c == 0 || c == nc)) {
-          // a face with finer neighbours: their averaged fluxes
-          // (boundary_fluxes, boundaries.F90:494-1060)
-          const int fs = a.ffix[b * 6 + 2 * DIR + (c == nc)];
-          if (fs >= 0) {
-            const int nf = (ND == 3) ? nc * nc : nc;
-#pragma unroll
-            for (int p = 0; p < NV; p++) f[p] = T(a.FB[((size_t)fs * NV + p) * nf + t]);
-          }
-        }
-        if (c >= 1) {
-          // cell c-1 has both faces
-          int i, j, k;
-          coords(c - 1, i, j, k);
-          const size_t bb = (size_t)b * NV * (size_t)rc.ncell;
-          const size_t bt = bb + (size_t)lidx<sizeof(T)>(nc, ND, i, j, k);
-          const size_t bd = bb + (size_t)lidx<8>(nc, ND, i, j, k);
-          const size_t bf = bb + (size_t)lidx<4>(nc, ND, i, j, k);
-          const T dxi = T(a.blev ? R->dxi[DIR] * double(1 << a.blev[b]) : R->dxi[DIR]);
-          double unew[NV];
-#pragma unroll
-          for (int v = 0; v < NV; v++) {
-            const size_t off = (size_t)v * rc.ncell;
-            // update_increment order: -dxi*dfx - dyi*dfy - dzi*dfz
-            const T dfx = f[v] - fprev[v];
-            T du;
-            if constexpr (DIR == 0) du = -dxi * dfx;
-            else if constexpr (kDin) du = sd[(((c - 1) & 3) * NV + v) * wg + tid] - dxi * dfx;
-            else du = dpre[v] - dxi * dfx;
-            if constexpr (kLast) {
-              // gravity (update_sources, sources.F90:288-335): du(m) += rho g,
-              // du(E) += rho g . v with g = (0, gacc, 0), zero terms included
-              if (rc.grav) {
-#pragma clang fp contract(off)
-                const T* Qg = static_cast<const T*>(a.Qold);
-                const size_t n1 = (size_t)rc.ncell;
-                const T rho = Qg[bt + (size_t)P::idn * n1];
-                const T gx = rho * T(0), gy = rho * T(rc.gacc), gz = rho * T(0);
-                if (v == P::imx) du = du + gx;
-                if (v == P::imy) du = du + gy;
-                if (ND == 3 && v == P::imz) du = du + gz;
-                if (v == P::ien) {
-                  du = (du + gx * Qg[bt + (size_t)P::ivx * n1]) + gy * Qg[bt + (size_t)P::ivy * n1];
-                  if (ND == 3) du = du + gz * Qg[bt + (size_t)P::ivz * n1];
-                }
-              }
-              // viscous source terms after the completed increment
-              // (update_sources, sources.F90:340-467; products of k_visc_src)
-              if (a.vsrc && (a.vis & 1)) {
-#pragma clang fp contract(off)
-                const T* V = static_cast<const T*>(a.vsrc) + (size_t)b * 9 * rc.ncell + (bt - bb);
-                const size_t n1 = (size_t)rc.ncell;
-                if (v == P::imx) du = du + V[0];
-                if (v == P::imy) du = du + V[n1];
-                if (v == P::imz) du = du + V[2 * n1];
-                if (v == P::ien) du = du + V[3 * n1];
-              }
-            }
-            if constexpr (kLast && P::mhd) {
-              // GLM source terms after the completed increment
-              // (update_sources, sources.F90:479-539; products from k_glm_src)
-              if (a.src) {
-#pragma clang fp contract(off)
-                const T* Sp = static_cast<const T*>(a.src) + (size_t)b * 8 * rc.ncell + (bt - bb);
-                const size_t n1 = (size_t)rc.ncell;
-                if (v == P::imx) du = du - Sp[0];
-                if (v == P::imy) du = du - Sp[n1];
-                if (v == P::imz) du = du - Sp[2 * n1];
-                if (v == P::ien) du = du - Sp[3 * n1];
-                if (a.glm > 1) {
-                  if (v == P::ibx) du = du - Sp[4 * n1];
-                  if (v == P::iby) du = du - Sp[5 * n1];
-                  if (v == P::ibz) du = du - Sp[6 * n1];
-                  if (v == P::ien) du = du - Sp[7 * n1];
-                }
-              }
-              // resistive source terms after the GLM ones (sources.F90:543-598)
-              if (a.vsrc && (a.vis & 2)) {
-#pragma clang fp contract(off)
-                const T* V = static_cast<const T*>(a.vsrc) + (size_t)b * 9 * rc.ncell + (bt - bb);
-                const size_t n1 = (size_t)rc.ncell;
-                if (v == P::ibx) du = du + V[4 * n1];
-                if (v == P::iby) du = du + V[5 * n1];
-                if (v == P::ibz) du = du + V[6 * n1];
-                if (v == P::ien) du = (du + V[7 * n1]) + V[8 * n1];
-              }
-            }
-            if constexpr (!kLast) {
-              if constexpr (kDout) sd[(((c - 1) & 3) * NV + v) * wg + tid] = du;
-              else Dp[bt + off] = du;
-            } else if constexpr (sizeof(T) == 8) {
-              double un = combine(a.kind, u0pre[v], u1pre[v], ds, du, a.ca, a.cb);
-              if (a.last && v == P::ibp) un = rc.decay * un;
-              unew[v] = un;
-            } else {
-              // mixed precision: the FP32 increment is added to the FP64
-              // state in increment form with Kahan compensation.  The true
-              // step state is U0 - C; a stage that writes the step state
-              // forms U0_true + delta and keeps the rounding error of that
-              // sum in C (the stages into U1 use U0 alone).
-              const double u0 = u0pre[v];
-              const double cp = double(cpre[v]);
-              const double dd = ds * double(du);
-              const double y =
-                  combine_delta(a.kind, u0, u1pre[v], cp, dd, a.ca, a.cb) - cp;
-              double un = u0 + y;
-              if (a.comp) {
-                double cn = (un - u0) - y;
-                if (a.last && v == P::ibp) { un = rc.decay * un; cn = rc.decay * cn; }
-                a.C[bf + off] = float(cn);
-              }
-              unew[v] = un;
-            }
-          }
-          if constexpr (kLast) {
-            double qn[NV];
-            if constexpr (P::sr) {
-              const int cs = cons2prim_sr<P>(rc.sc, unew, qn);
-              if (cs) {
-                c2p_keep_old<P, T>(cs, qn, static_cast<const T*>(a.Qold), bt, rc.ncell);
-                c2p_count(a.st, cs);
-              }
-            } else {
-              cons2prim<P, double>(ed, unew, qn);
-            }
-#pragma unroll
-            for (int v = 0; v < NV; v++) {
-              const size_t off = (size_t)v * rc.ncell;
-              a.Uout[bd + off] = unew[v];
-              Qo[bt + off] = T(qn[v]);
-            }
-            if (a.last) smax = fmax(smax, maxspeed<P, double>(ed, qn));
-          }
-        }
-        if constexpr (kDout) {
-          if (c >= 1 && ((c - 1) & 3) == 3) {
-            size_t base[4];
-            dchunk_base(c - 4, base);
-#pragma unroll
-            for (int m = 0; m < 4; m++)
-#pragma unroll
-              for (int v = 0; v < NV; v++)
-                Dp[base[m] + (size_t)v * rc.ncell] = sd[(m * NV + v) * wg + tid];
-          }
-        }
-#pragma unroll
-        for (int p = 0; p < NV; p++) fprev[p] = f[p];
-      }
-#pragma unroll
-      for (int p = 0; p < NV; p++) flp[p] = flc[p];
     }
   }
+  if constexpr (R > 0) __syncthreads();   // the face states replace the cells
+  if (active && c < nc) {
+#pragma unroll
+    for (int v = 0; v < NV; v++) face[v * nf + p * wf + c + 1] = flc[v];
+  }
+  __syncthreads();
+  T ql[NV];
+  if (active && c >= 0) {
+#pragma unroll
+    for (int v = 0; v < NV; v++) ql[v] = face[rot<P, DIR>(v) * nf + p * wf + c];
+  }
+  __syncthreads();   // the fluxes replace the face states
+  if (active && c >= 0) {
+    // face c-1/2: left state from cell c-1, right state from cell c
+    T qr[NV], fr[NV];
+#pragma unroll
+    for (int v = 0; v < NV; v++) qr[v] = frc[rot<P, DIR>(v)];
+    riemann<P, RS, T>(e, rc.sc, cmax, cmax2, ql, qr, fr);
+#pragma unroll
+    for (int v = 0; v < NV; v++) f[rot<P, DIR>(v)] = fr[v];
+    if (a.ffix && (c == 0 || c == nc)) {
+      // a face with finer neighbours: their averaged fluxes
+      // (boundary_fluxes, boundaries.F90:494-1060)
+      const int fs = a.ffix[b * 6 + 2 * DIR + (c == nc)];
+      if (fs >= 0) {
+#pragma unroll
+        for (int v = 0; v < NV; v++)
+          f[v] = T(a.FB[((size_t)fs * NV + v) * npen + c1 + nc * c2]);
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < NV; v++) face[v * nf + p * wf + c] = f[v];
+  }
+  __syncthreads();
+  if (inner) {
+    const unsigned od = ob + lidx<8>(nc, ND, ci, cj, ck), of = ob + lidx<4>(nc, ND, ci, cj, ck);
+    const unsigned oc = ot - ob;      // the cell inside its block
+    T* __restrict__ Dp = static_cast<T*>(a.D) + base0;
+    T* __restrict__ Qo = static_cast<T*>(a.Qout) + base0;
+    const double* U0 = a.U0 + base0;
+    const double* U1 = a.U1 + base0;
+    double* Uo = a.Uout + base0;
+    float* Cp = sizeof(T) == 4 ? a.C + base0 : nullptr;
+    T dpre[NV], fn[NV];
+    double u0pre[NV], u1pre[NV];
+    float cpre[NV];
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      const int off = v * rc.ncell;
+      if constexpr (DIR > 0) dpre[v] = at_byte(Dp + off, ot * (unsigned)sizeof(T));
+      if constexpr (kLast) {
+        u0pre[v] = at_byte(U0 + off, od * 8u);
+        if (a.kind != 0) u1pre[v] = at_byte(U1 + off, od * 8u);
+        // the compensation enters the updates of the step state; the
+        // transient stages ignore it (it is below the FP64 rounding of U0)
+        if constexpr (sizeof(T) == 4) cpre[v] = a.comp ? at_byte(Cp + off, of * 4u) : 0.0f;
+      }
+      fn[v] = face[v * nf + p * wf + c + 1];
+    }
+    const double ds = kLast ? a.fac * dt_of(rc, Rs, a.slot, a.dtnext) : 0.0;
+    const EosConst<double> ed{rc.gamma, rc.gammam1, rc.gammam1i, rc.csnd, rc.csnd2};
+    const T dxi = T(a.blev ? Rs->dxi[DIR] * double(1 << a.blev[b]) : Rs->dxi[DIR]);
+    double unew[NV];
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      const int off = v * rc.ncell;
+      // update_increment order: -dxi*dfx - dyi*dfy - dzi*dfz
+      const T dfx = fn[v] - f[v];
+      T du;
+      if constexpr (DIR == 0) du = -dxi * dfx;
+      else du = dpre[v] - dxi * dfx;
+      if constexpr (kLast) {
+        // gravity (update_sources, sources.F90:288-335): du(m) += rho g,
+        // du(E) += rho g . v with g = (0, gacc, 0), zero terms included
+        if (rc.grav) {
+#pragma clang fp contract(off)
+          const T* Qg = static_cast<const T*>(a.Qold);
+          const size_t n1 = (size_t)rc.ncell;
+          const T rho = Qg[base0 + ot + (size_t)P::idn * n1];
+          const T gx = rho * T(0), gy = rho * T(rc.gacc), gz = rho * T(0);
+          if (v == P::imx) du = du + gx;
+          if (v == P::imy) du = du + gy;
+          if (ND == 3 && v == P::imz) du = du + gz;
+          if (v == P::ien) {
+            du = (du + gx * Qg[base0 + ot + (size_t)P::ivx * n1]) + gy * Qg[base0 + ot + (size_t)P::ivy * n1];
+            if (ND == 3) du = du + gz * Qg[base0 + ot + (size_t)P::ivz * n1];
+          }
+        }
+        // viscous source terms after the completed increment
+        // (update_sources, sources.F90:340-467; products of k_visc_src)
+        if (a.vsrc && (a.vis & 1)) {
+#pragma clang fp contract(off)
+          const T* V = static_cast<const T*>(a.vsrc) + (size_t)b * 9 * rc.ncell + oc;
+          const size_t n1 = (size_t)rc.ncell;
+          if (v == P::imx) du = du + V[0];
+          if (v == P::imy) du = du + V[n1];
+          if (v == P::imz) du = du + V[2 * n1];
+          if (v == P::ien) du = du + V[3 * n1];
+        }
+      }
+      if constexpr (kLast && P::mhd) {
+        // GLM source terms after the completed increment
+        // (update_sources, sources.F90:479-539; products from k_glm_src)
+        if (a.src) {
+#pragma clang fp contract(off)
+          const T* Sp = static_cast<const T*>(a.src) + (size_t)b * 8 * rc.ncell + oc;
+          const size_t n1 = (size_t)rc.ncell;
+          if (v == P::imx) du = du - Sp[0];
+          if (v == P::imy) du = du - Sp[n1];
+          if (v == P::imz) du = du - Sp[2 * n1];
+          if (v == P::ien) du = du - Sp[3 * n1];
+          if (a.glm > 1) {
+            if (v == P::ibx) du = du - Sp[4 * n1];
+            if (v == P::iby) du = du - Sp[5 * n1];
+            if (v == P::ibz) du = du - Sp[6 * n1];
+            if (v == P::ien) du = du - Sp[7 * n1];
+          }
+        }
+        // resistive source terms after the GLM ones (sources.F90:543-598)
+        if (a.vsrc && (a.vis & 2)) {
+#pragma clang fp contract(off)
+          const T* V = static_cast<const T*>(a.vsrc) + (size_t)b * 9 * rc.ncell + oc;
+          const size_t n1 = (size_t)rc.ncell;
+          if (v == P::ibx) du = du + V[4 * n1];
+          if (v == P::iby) du = du + V[5 * n1];
+          if (v == P::ibz) du = du + V[6 * n1];
+          if (v == P::ien) du = (du + V[7 * n1]) + V[8 * n1];
+        }
+      }
+      if constexpr (!kLast) {
+        at_byte(Dp + off, ot * (unsigned)sizeof(T)) = du;
+      } else if constexpr (sizeof(T) == 8) {
+        double un = combine(a.kind, u0pre[v], u1pre[v], ds, du, a.ca, a.cb);
+        if (a.last && v == P::ibp) un = rc.decay * un;
+        unew[v] = un;
+      } else {
+        // mixed precision: the FP32 increment is added to the FP64
+        // state in increment form with Kahan compensation.  The true
+        // step state is U0 - C; a stage that writes the step state
+        // forms U0_true + delta and keeps the rounding error of that
+        // sum in C (the stages into U1 use U0 alone).
+        const double u0 = u0pre[v];
+        const double cp = double(cpre[v]);
+        const double dd = ds * double(du);
+        const double y =
+            combine_delta(a.kind, u0, u1pre[v], cp, dd, a.ca, a.cb) - cp;
+        double un = u0 + y;
+        if (a.comp) {
+          double cn = (un - u0) - y;
+          if (a.last && v == P::ibp) { un = rc.decay * un; cn = rc.decay * cn; }
+          at_byte(Cp + off, of * 4u) = float(cn);
+        }
+        unew[v] = un;
+      }
+    }
+    if constexpr (kLast) {
+      double qn[NV];
+      if constexpr (P::sr) {
+        const int cs = cons2prim_sr<P>(rc.sc, unew, qn);
+        if (cs) {
+          c2p_keep_old<P, T>(cs, qn, static_cast<const T*>(a.Qold), base0 + ot, rc.ncell);
+          c2p_count(a.st, cs);
+        }
+      } else {
+        cons2prim<P, double>(ed, unew, qn);
+      }
+#pragma unroll
+      for (int v = 0; v < NV; v++) {
+        const int off = v * rc.ncell;
+        at_byte(Uo + off, od * 8u) = unew[v];
+        at_byte(Qo + off, ot * (unsigned)sizeof(T)) = T(qn[v]);
+      }
+      if (a.last) smax = fmax(smax, maxspeed<P, double>(ed, qn));
+    }
+  }
+  return smax;
+}
 
+// One sweep: the workgroup's pencils are np consecutive ones of the pool.
+template <class P, int REC, int RS, int ND, int DIR, typename T>
+__global__ __launch_bounds__(512, (sweep_min_waves<P, RS, T>()))
+void k_sweep(SweepArgs a, RunConst rc) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  constexpr bool kLast = DIR == ND - 1;
+  reset_speed(a, rc);
+  int run;
+  const double smax = sweep_cells<P, REC, RS, ND, DIR, T>(
+      a, rc, workgroup_index(a.swz) * a.np, a.np, reinterpret_cast<T*>(smem), run);
   if constexpr (kLast) {
     if (a.last) wg_max_speed(a.rs, a.spart, run, a.slot ^ 1, smax);
-  }
-}
-
-template <class P, int REC, int RS, int ND, int DIR, typename T>
-__global__ __launch_bounds__(256, sweep_min_waves<T>()) void k_sweep(SweepArgs a, RunConst rc) {
-  sweep_body<P, REC, RS, ND, DIR, T>(a, rc);
-}
-
-// One launch per stage: when a workgroup's pencils are whole blocks in
-// every direction (npen divides the workgroup size), the sweeps of one
-// block depend only on each other through its own increment D (each
-// direction reads the stage input Q, including the neighbours' halo, which
-// no sweep of the stage writes), so one workgroup runs its blocks' x, y (and
-// z) sweeps in turn with a workgroup barrier between them; D stays in the
-// caches between the directions.
-template <class P, int REC, int RS, int ND, typename T>
-__global__ __launch_bounds__(256, sweep_min_waves<T>()) void k_stage(SweepArgs a, RunConst rc) {
-  sweep_body<P, REC, RS, ND, 0, T>(a, rc);
-  __syncthreads();
-  a.first = 0;
-  sweep_body<P, REC, RS, ND, 1, T>(a, rc);
-  if constexpr (ND == 3) {
-    __syncthreads();
-    sweep_body<P, REC, RS, ND, 2, T>(a, rc);
   }
 }
 
@@ -1580,20 +1631,6 @@ static __global__ void k_zero_f32(float* x, long long n) {
 static __global__ void k_reset_slot(RunState* rs, int slot, int r0, int nr) {
   const int r = r0 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (r < r0 + nr) rs[r].cmax_bits[slot] = (unsigned long long)__double_as_longlong(kTiny);
-}
-
-// end of a step, one thread per run: dt into the trace ring
-// trace[(step mod tsteps) * nruns + run], time and step advanced
-static __global__ void k_end_step(RunState* rs, double* trace, int tsteps, RunConst rc, int slot,
-                           double dtnext) {
-  const int r = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (r >= rc.nruns) return;
-  RunState* R = rs + r;
-  const double dt = dt_of(rc, R, slot, dtnext);
-  trace[(size_t)(R->step % tsteps) * rc.nruns + r] = dt;
-  R->dt = dt;
-  R->time += dt;
-  R->step += 1;
 }
 
 // dt of the current slot without advancing (new_time_step alone), per run:
@@ -1883,7 +1920,8 @@ using namespace amun_dev;
 // kernel instantiations selected for one configuration
 struct Dispatch {
   SweepFn sweep[3] = {nullptr, nullptr, nullptr};
-  SweepFn stage = nullptr;   // all directions of a stage in one launch (k_stage)
+    int R = 0;                 // window half width of the reconstruction
+  bool stage = false;        // set_stage_fusion is accepted
   void (*compact[3])(const void*, const int*, RunConst, DevState*) = {nullptr, nullptr, nullptr};
   void (*prim)(const double*, void*, RunConst, DevState*, RunState*, const int*, int, int,
                int) = nullptr;
@@ -1925,12 +1963,11 @@ void fill(Dispatch& d) {
     d.compact[1] = k_compact<P, REC, ND, 1, T>;
     if constexpr (ND == 3) d.compact[2] = k_compact<P, REC, ND, 2, T>;
   }
+  d.R = Recon<P, REC, ND, 0, T>::R;
+  d.stage = (REC == REC_TVD || REC == REC_WENO5Z) && !P::sr;
   d.sweep[0] = k_sweep<P, REC, RS, ND, 0, T>;
   d.sweep[1] = k_sweep<P, REC, RS, ND, 1, T>;
   if constexpr (ND == 3) d.sweep[2] = k_sweep<P, REC, RS, ND, 2, T>;
-  // the fused stage for the reconstructions of the production workloads
-  if constexpr ((REC == REC_TVD || REC == REC_WENO5Z) && !P::sr)
-    d.stage = k_stage<P, REC, RS, ND, T>;
   d.prim = k_prim<P, T>;
   d.integ = k_integrals<P>;
   d.stats = k_stats<P, T>;
