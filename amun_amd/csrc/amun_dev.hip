@@ -6,6 +6,7 @@
 #include "kernels.h"
 #include "remesh.h"
 #include "sources.h"
+#include "transfer.h"
 
 #include <array>
 #include <map>
@@ -1069,106 +1070,117 @@ static int after_upload(amun_ctx* c, int r0, int nr, bool zero_c = true) {
   return 0;
 }
 
-// global array U[nv][nz][ny][nx] of run r <-> its blocks (h: the run's
-// segment of the pool, FP64 layout of lidx<8>)
-static void scatter_run(const amun_ctx* c, int r, const double* u, double* h) {
-  const RunConst& rc = c->rc;
-  const int nc = rc.nc, nv = c->nv, b0 = c->run_b0[r], b1 = c->run_b0[r + 1];
-  const amun_grid& G = c->grids[r];
-  const size_t nx = (size_t)G.xblocks * nc, ny = (size_t)G.yblocks * nc;
-  const size_t nz = (rc.nd == 3) ? (size_t)G.zblocks * nc : 1;
-  const int kn = (rc.nd == 3) ? nc : 1;
-  for (int b = b0; b < b1; b++) {
-    const size_t bx = c->coords[b * 3], by = c->coords[b * 3 + 1], bz = c->coords[b * 3 + 2];
-    for (int v = 0; v < nv; v++)
-      for (int k = 0; k < kn; k++)
-        for (int j = 0; j < nc; j++) {
-          const double* src = u + ((v * nz + bz * kn + k) * ny + by * nc + j) * nx + bx * nc;
-          double* dst = &h[((size_t)(b - b0) * nv + v) * rc.ncell];
-          for (int i = 0; i < nc; i++) dst[lidx<8>(nc, rc.nd, i, j, k)] = src[i];
-        }
-  }
+// Between steps U1 holds nothing (the first stage of every integrator writes
+// it), so the transfers convert in it and allocate nothing.
+static dim3 transfer_grid(long long n) {
+  return dim3((unsigned)std::max(1ll, std::min(8192ll, (n + 255) / 256)));
 }
 
-static void gather_run(const amun_ctx* c, int r, const double* h, double* u, int es) {
-  const RunConst& rc = c->rc;
-  const int nc = rc.nc, nv = c->nv, b0 = c->run_b0[r], b1 = c->run_b0[r + 1];
+static GridShape run_shape(const amun_ctx* c, int r) {
   const amun_grid& G = c->grids[r];
-  const size_t nx = (size_t)G.xblocks * nc, ny = (size_t)G.yblocks * nc;
-  const size_t nz = (rc.nd == 3) ? (size_t)G.zblocks * nc : 1;
-  const int kn = (rc.nd == 3) ? nc : 1;
-  for (int b = b0; b < b1; b++) {
-    const size_t bx = c->coords[b * 3], by = c->coords[b * 3 + 1], bz = c->coords[b * 3 + 2];
-    for (int v = 0; v < nv; v++)
-      for (int k = 0; k < kn; k++)
-        for (int j = 0; j < nc; j++) {
-          double* dst = u + ((v * nz + bz * kn + k) * ny + by * nc + j) * nx + bx * nc;
-          const double* src = &h[((size_t)(b - b0) * nv + v) * rc.ncell];
-          if (es == 8)
-            for (int i = 0; i < nc; i++) dst[i] = src[lidx<8>(nc, rc.nd, i, j, k)];
-          else
-            for (int i = 0; i < nc; i++) dst[i] = src[lidx<4>(nc, rc.nd, i, j, k)];
-        }
-  }
+  return {c->run_b0[r], G.xblocks, G.yblocks, c->rc.nd == 3 ? G.zblocks : 1};
 }
 
-// Multi-level meshes: interiors of u from U0, q with its ghost layers
-// (virtual blocks filled from the current state), and the ghost layers of u
-// as prim2cons of q's (update_ghost_cells, boundaries.F90:6633-6736).
-static int download_blocks_amr(amun_ctx* c, double* u, double* q) {
-  const RunConst& rc = c->rc;
-  const int ng = c->cfg.nghosts, nc = rc.nc, nv = c->nv, nd = rc.nd;
-  const int im = nc + 2 * ng, km = (nd == 3) ? im : 1, kg = (nd == 3) ? ng : 0;
-  const size_t per = (size_t)im * im * km;
-  int r = c->amr.on ? amr_fill(c, c->qcur, (int)(c->nsteps & 1)) : bnd_fill(c, c->qcur);
-  if (r) return r;
-  const size_t n = (size_t)rc.nblk * per * nv;
-  std::vector<double> qh(n);
-  double* buf = nullptr;
-  HIP_TRY(hipMalloc((void**)&buf, n * sizeof(double)));
-  hipLaunchKernelGGL(c->disp.pack_q, dim3(2048), dim3(256), 0, c->stream,
-                     (const void*)c->Q[c->qcur], buf, c->nbr, rc, ng);
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-  if (e == hipSuccess) e = hipMemcpy(qh.data(), buf, n * sizeof(double), hipMemcpyDeviceToHost);
-  hipFree(buf);
-  if (e != hipSuccess) return fail(1000 + (int)e, "download_blocks");
-  std::vector<double> h(c->nstate);
-  HIP_TRY(hipMemcpy(h.data(), c->U0, c->nstate * sizeof(double), hipMemcpyDeviceToHost));
-  const bool mhd = has_field(c->cfg), iso = c->cfg.eos == AMUN_EOS_ISO;
-  const double g1 = c->cfg.gamma - 1.0;
-  for (int b = 0; b < rc.nblk; b++)
-    for (int k = 0; k < km; k++)
-      for (int j = 0; j < im; j++)
-        for (int i = 0; i < im; i++) {
-          const size_t cell = (size_t)b * per + ((size_t)k * im + j) * im + i;
-          double* uo = u + cell * nv;
-          const double* qq = qh.data() + cell * nv;
-          const int li = i - ng, lj = j - ng, lk = k - kg;
-          if (li >= 0 && li < nc && lj >= 0 && lj < nc && lk >= 0 && lk < (nd == 3 ? nc : 1)) {
-            for (int v = 0; v < nv; v++)
-              uo[v] = h[((size_t)b * nv + v) * rc.ncell + lidx<8>(nc, nd, li, lj, lk)];
-          } else {
-            // prim2cons_hd_adi / prim2cons_mhd_adi (equations.F90:1762, 2815)
-            uo[0] = qq[0];
-            uo[1] = qq[0] * qq[1];
-            uo[2] = qq[0] * qq[2];
-            uo[3] = qq[0] * qq[3];
-            const double ek = 0.5 * ((uo[1] * qq[1] + uo[2] * qq[2]) + uo[3] * qq[3]);
-            if (iso) {
-              // prim2cons_hd_iso / _mhd_iso (equations.F90:1360, 2220)
-              for (int v = 4; v < nv; v++) uo[v] = qq[v];
-            } else if (mhd) {
-              for (int v = 4; v < 8; v++) uo[v] = qq[v];
-              const double em = 0.5 * ((qq[4] * qq[4] + qq[5] * qq[5]) + qq[6] * qq[6]);
-              uo[8] = (qq[8] / g1 + ek) + em;
-            } else {
-              uo[4] = qq[4] / g1 + ek;
-            }
-          }
-        }
-  if (q) std::memcpy(q, qh.data(), n * sizeof(double));
+// the global array U[nv][nz][ny][nx] of run r on the host into the pool X of
+// FP64 block arrays
+static int grid_to_pool(amun_ctx* c, int r, const double* u, double* X) {
+  const size_t per = (size_t)c->nv * c->rc.ncell;
+  const long long n = (long long)(c->run_b0[r + 1] - c->run_b0[r]) * c->rc.ncell;
+  HIP_TRY(hipMemcpyAsync(c->U1, u, (size_t)n / c->rc.ncell * per * sizeof(double),
+                         hipMemcpyHostToDevice, c->stream));
+  hipLaunchKernelGGL((k_grid_transfer<double, true>), dim3(transfer_grid(n).x, c->nv), dim3(256),
+                     0, c->stream, X, (const double*)c->U1, run_shape(c, r), c->rc, c->nv);
+  HIP_TRY(hipGetLastError());
   return 0;
+}
+
+// run r of the pool X (element size es) into the global array u on the host
+static int pool_to_grid(amun_ctx* c, int r, const void* X, size_t es, double* u) {
+  const size_t per = (size_t)c->nv * c->rc.ncell;
+  const long long n = (long long)(c->run_b0[r + 1] - c->run_b0[r]) * c->rc.ncell;
+  const dim3 grid(transfer_grid(n).x, c->nv);
+  if (es == sizeof(double))
+    hipLaunchKernelGGL((k_grid_transfer<double, false>), grid, dim3(256), 0, c->stream,
+                       static_cast<const double*>(X), c->U1, run_shape(c, r), c->rc, c->nv);
+  else
+    hipLaunchKernelGGL((k_grid_transfer<float, false>), grid, dim3(256), 0, c->stream,
+                       static_cast<const float*>(X), c->U1, run_shape(c, r), c->rc, c->nv);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipMemcpyAsync(u, c->U1, (size_t)n / c->rc.ncell * per * sizeof(double),
+                         hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  return 0;
+}
+
+// Calls f(buffer, first block, blocks) over all blocks, with a device buffer
+// of per doubles a block: U1 for as many blocks as it holds, or, where it
+// holds none (ghost layers around few small blocks), an allocation for all.
+extern "C++" template <class F>
+static int by_block_chunks(amun_ctx* c, size_t per, F&& f) {
+  const int nblk = c->rc.nblk;
+  if (c->nstate < per) {
+    double* buf = nullptr;
+    HIP_TRY(hipMalloc((void**)&buf, nblk * per * sizeof(double)));
+    const int r = f(buf, 0, nblk);
+    HIP_TRY(hipFree(buf));
+    return r;
+  }
+  const int m = (int)std::min<size_t>(nblk, c->nstate / per);
+  int r = 0;
+  for (int b0 = 0; b0 < nblk && !r; b0 += m) r = f(c->U1, b0, std::min(m, nblk - b0));
+  return r;
+}
+
+// the conserved state of all blocks to or from arrays of m^d cells a block
+// with ng cells before the interior (k_block_transfer)
+static int blocks_to_pool(amun_ctx* c, const double* u, int m, int ng) {
+  const size_t per = (size_t)c->nv * m * m * (c->rc.nd == 3 ? m : 1);
+  return by_block_chunks(c, per, [&](double* buf, int b0, int nb) -> int {
+    HIP_TRY(hipMemcpyAsync(buf, u + b0 * per, nb * per * sizeof(double), hipMemcpyHostToDevice,
+                           c->stream));
+    hipLaunchKernelGGL((k_block_transfer<true>),
+                       transfer_grid((long long)nb * c->nv * c->rc.ncell), dim3(256), 0,
+                       c->stream, c->U0, (const double*)buf, b0, nb, m, ng, c->rc, c->nv);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    return 0;
+  });
+}
+
+// Block arrays with ghost layers where ghosts come from virtual blocks
+// (multi-level meshes, non-periodic sides): u from U0 and, in the ghost
+// layers, prim2cons of q's; q from the primitive pool filled from the
+// current state.
+static int download_blocks_virtual(amun_ctx* c, double* u, double* q) {
+  const RunConst& rc = c->rc;
+  const int ng = c->cfg.nghosts, im = rc.nc + 2 * ng;
+  const size_t per = (size_t)c->nv * im * im * (rc.nd == 3 ? im : 1);
+  int r = c->amr.on ? amr_fill(c, c->qcur, (int)(c->nsteps & 1)) : bnd_fill(c, c->qcur);
+  for (int pass = 0; pass < 2 && !r; pass++) {
+    double* dst = pass == 0 ? u : q;
+    if (!dst) continue;
+    const double* U = pass == 0 ? c->U0 : nullptr;
+    r = by_block_chunks(c, per, [&](double* buf, int b0, int nb) -> int {
+      const dim3 grid = transfer_grid((long long)(nb * per / c->nv));
+      by_system(c->cfg, [&](auto tag) {
+        using P = decltype(tag);
+        if (c->qsize == sizeof(double))
+          hipLaunchKernelGGL((k_blocks_ghosts<P, double>), grid, dim3(256), 0, c->stream,
+                             static_cast<const double*>(c->Q[c->qcur]), U, buf, c->nbr, rc, ng,
+                             b0, nb);
+        else
+          hipLaunchKernelGGL((k_blocks_ghosts<P, float>), grid, dim3(256), 0, c->stream,
+                             static_cast<const float*>(c->Q[c->qcur]), U, buf, c->nbr, rc, ng,
+                             b0, nb);
+      });
+      HIP_TRY(hipGetLastError());
+      HIP_TRY(hipMemcpyAsync(dst + b0 * per, buf, nb * per * sizeof(double),
+                             hipMemcpyDeviceToHost, c->stream));
+      HIP_TRY(hipStreamSynchronize(c->stream));
+      return 0;
+    });
+  }
+  return r;
 }
 
 int amun_dev_upload_run(amun_ctx* c, int32_t r, const double* u) {
@@ -1176,14 +1188,8 @@ int amun_dev_upload_run(amun_ctx* c, int32_t r, const double* u) {
   if (c->amr.on)
     return fail(600, "multi-level meshes transfer block arrays (amun_dev_upload_blocks)");
   if (r < 0 || r >= c->rc.nruns) return fail(500, "run index out of range");
-  const size_t per = (size_t)c->nv * c->rc.ncell;
-  const size_t n = (size_t)(c->run_b0[r + 1] - c->run_b0[r]) * per;
-  std::vector<double> h(n);
-  scatter_run(c, r, u, h.data());
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  HIP_TRY(hipMemcpy(c->U0 + (size_t)c->run_b0[r] * per, h.data(), n * sizeof(double),
-                    hipMemcpyHostToDevice));
-  return after_upload(c, r, 1);
+  const int e = grid_to_pool(c, r, u, c->U0);
+  return e ? e : after_upload(c, r, 1);
 }
 
 int amun_dev_upload_global(amun_ctx* c, const double* u) {
@@ -1194,22 +1200,30 @@ int amun_dev_upload_global(amun_ctx* c, const double* u) {
 
 int amun_dev_upload_blocks(amun_ctx* c, const double* u) {
   if (!c || !u) return fail(500, "null argument");
-  const RunConst& rc = c->rc;
-  const int nc = rc.nc, nv = c->nv, ng = c->cfg.nghosts;
-  const int im = nc + 2 * ng, km = (rc.nd == 3) ? im : 1, kn = (rc.nd == 3) ? nc : 1;
-  const int kg = (rc.nd == 3) ? ng : 0;
-  const size_t per = (size_t)nv * im * im * km;
-  std::vector<double> h(c->nstate);
-  for (int b = 0; b < rc.nblk; b++)
-    for (int k = 0; k < kn; k++)
-      for (int j = 0; j < nc; j++)
-        for (int i = 0; i < nc; i++)
-          for (int v = 0; v < nv; v++)
-            h[(((size_t)b * nv + v) * rc.ncell) + lidx<8>(nc, rc.nd, i, j, k)] =
-                u[b * per + ((((size_t)(k + kg) * im + (j + ng)) * im + (i + ng)) * nv) + v];
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  HIP_TRY(hipMemcpy(c->U0, h.data(), c->nstate * sizeof(double), hipMemcpyHostToDevice));
-  return after_upload(c, 0, rc.nruns);
+  const int ng = c->cfg.nghosts;
+  const int e = blocks_to_pool(c, u, c->rc.nc + 2 * ng, ng);
+  return e ? e : after_upload(c, 0, c->rc.nruns);
+}
+
+int amun_dev_upload_interiors(amun_ctx* c, const double* u) {
+  if (!c || !u) return fail(500, "null argument");
+  const int e = blocks_to_pool(c, u, c->rc.nc, 0);
+  return e ? e : after_upload(c, 0, c->rc.nruns);
+}
+
+int amun_dev_download_interiors(amun_ctx* c, double* u) {
+  if (!c || !u) return fail(500, "null argument");
+  const size_t per = (size_t)c->nv * c->rc.ncell;
+  return by_block_chunks(c, per, [&](double* buf, int b0, int nb) -> int {
+    hipLaunchKernelGGL((k_block_transfer<false>), transfer_grid((long long)(nb * per)),
+                       dim3(256), 0, c->stream, (const double*)c->U0, buf, b0, nb, c->rc.nc, 0,
+                       c->rc, c->nv);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpyAsync(u + b0 * per, buf, nb * per * sizeof(double), hipMemcpyDeviceToHost,
+                           c->stream));
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    return 0;
+  });
 }
 
 int amun_dev_download_run(amun_ctx* c, int32_t r, double* u, double* q) {
@@ -1217,27 +1231,8 @@ int amun_dev_download_run(amun_ctx* c, int32_t r, double* u, double* q) {
   if (c->amr.on)
     return fail(600, "multi-level meshes transfer block arrays (amun_dev_download_blocks)");
   if (r < 0 || r >= c->rc.nruns) return fail(500, "run index out of range");
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  const size_t per = (size_t)c->nv * c->rc.ncell;
-  const size_t off = (size_t)c->run_b0[r] * per;
-  const size_t n = (size_t)(c->run_b0[r + 1] - c->run_b0[r]) * per;
-  std::vector<double> h(n);
-  HIP_TRY(hipMemcpy(h.data(), c->U0 + off, n * sizeof(double), hipMemcpyDeviceToHost));
-  gather_run(c, r, h.data(), u, 8);
-  if (q) {
-    if (c->qsize == sizeof(double)) {
-      HIP_TRY(hipMemcpy(h.data(), (const double*)c->Q[c->qcur] + off, n * sizeof(double),
-                        hipMemcpyDeviceToHost));
-      gather_run(c, r, h.data(), q, 8);
-    } else {
-      std::vector<float> hf(n);
-      HIP_TRY(hipMemcpy(hf.data(), (const float*)c->Q[c->qcur] + off, n * sizeof(float),
-                        hipMemcpyDeviceToHost));
-      for (size_t m = 0; m < n; m++) h[m] = hf[m];
-      gather_run(c, r, h.data(), q, 4);
-    }
-  }
-  return 0;
+  const int e = pool_to_grid(c, r, c->U0, sizeof(double), u);
+  return e || !q ? e : pool_to_grid(c, r, c->Q[c->qcur], c->qsize, q);
 }
 
 int amun_dev_download_global(amun_ctx* c, double* u, double* q) {
@@ -1249,7 +1244,7 @@ int amun_dev_download_global(amun_ctx* c, double* u, double* q) {
 int amun_dev_download_blocks(amun_ctx* c, double* u, double* q) {
   if (!c || !u) return fail(500, "null argument");
   // ghost layers from virtual blocks: u ghosts as prim2cons of q's
-  if (c->amr.on || c->bnd.on) return download_blocks_amr(c, u, q);
+  if (c->amr.on || c->bnd.on) return download_blocks_virtual(c, u, q);
   Dispatch& d = dispatch_of(c);
   const int ng = c->cfg.nghosts, nc = c->rc.nc;
   const int im = nc + 2 * ng, km = (c->rc.nd == 3) ? im : 1;
@@ -2348,18 +2343,14 @@ int recompute_segment(amun_ctx* c, int s0, int s1, double* seg) {
 
 // global array of the single run <-> pool layout (device buffer dst/src)
 int global_to_pool(amun_ctx* c, const double* g, double* dpool) {
-  std::vector<double> h(c->nstate);
-  scatter_run(c, 0, g, h.data());
-  HIP_TRY(hipMemcpy(dpool, h.data(), c->nstate * sizeof(double), hipMemcpyHostToDevice));
+  const int r = grid_to_pool(c, 0, g, dpool);
+  if (r) return r;
+  HIP_TRY(hipStreamSynchronize(c->stream));
   return 0;
 }
 
 int pool_to_global(amun_ctx* c, const double* dpool, double* g) {
-  std::vector<double> h(c->nstate);
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  HIP_TRY(hipMemcpy(h.data(), dpool, c->nstate * sizeof(double), hipMemcpyDeviceToHost));
-  gather_run(c, 0, h.data(), g, 8);
-  return 0;
+  return pool_to_grid(c, 0, dpool, sizeof(double), g);
 }
 
 }  // namespace

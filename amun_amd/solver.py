@@ -36,6 +36,7 @@ EXPORTS = (
     "amun_dev_tape_backward", "amun_dev_tape_tangent", "amun_dev_run_fixed",
     "amun_dev_init_amr", "amun_dev_amr_info", "amun_dev_statistics",
     "amun_dev_statistics_run", "amun_dev_set_stage_fusion",
+    "amun_dev_upload_interiors", "amun_dev_download_interiors",
 )
 
 
@@ -71,6 +72,8 @@ def load_library(path: str = LIB_PATH):
     L.amun_dev_upload_blocks.argtypes = [vp, _P]
     L.amun_dev_upload_global.argtypes = [vp, _P]
     L.amun_dev_download_blocks.argtypes = [vp, _P, _P]
+    L.amun_dev_upload_interiors.argtypes = [vp, _P]
+    L.amun_dev_download_interiors.argtypes = [vp, _P]
     L.amun_dev_download_global.argtypes = [vp, _P, _P]
     L.amun_dev_new_time_step.argtypes = [vp, ctypes.c_double, _P, _P]
     L.amun_dev_step.argtypes = [vp, ctypes.c_double, _P, _P]
@@ -424,25 +427,27 @@ class AmrSolver(Solver):
             return a[:, 0, g:g + p.ncells, g:g + p.ncells, :]
         return a[:, g:g + p.ncells, g:g + p.ncells, g:g + p.ncells, :]
 
+    def _interior_shape(self):
+        p = self.params
+        return (self.meta.shape[0],) + (p.ncells,) * p.ndims + (p.nv,)
+
     def upload(self, u: np.ndarray):
-        full = np.zeros(self._block_shape())
-        inner = self._interior(full)
-        inner[...] = np.asarray(u, dtype=np.float64).reshape(inner.shape)
-        self.upload_blocks(full)
+        u = np.ascontiguousarray(np.asarray(u, dtype=np.float64).reshape(self._interior_shape()))
+        self._check(self.lib.amun_dev_upload_interiors(self.h, _dp(u)))
 
     def download(self, with_q: bool = False):
         """Interiors of u (and q with its ghost layers, as after
         boundary_variables, if with_q)."""
-        if with_q:
-            u, q = self.download_blocks(with_q=True)
-        else:
-            u, q = self.download_blocks(), None
+        if not with_q:
+            ui = np.empty(self._interior_shape())
+            self._check(self.lib.amun_dev_download_interiors(self.h, _dp(ui)))
+            return ui
+        u, q = self.download_blocks(with_q=True)
         ui = np.ascontiguousarray(self._interior(u))
         if self.params.ndims == 2:
             ui = ui.reshape(ui.shape[0], self.params.ncells, self.params.ncells, -1)
-            if with_q:
-                q = q[:, 0]
-        return (ui, q) if with_q else ui
+            q = q[:, 0]
+        return ui, q
 
 
 class Batch(Solver):

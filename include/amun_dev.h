@@ -304,6 +304,13 @@ int  amun_dev_upload_global(amun_ctx* ctx, const double* u);
  * _blocks fills the ghost layers too, as after boundary_variables
  * (boundaries.F90:372-479), all runs of a batch; _global needs a single run. */
 int  amun_dev_download_blocks(amun_ctx* ctx, double* u, double* q);
+
+/* The conserved state of every block's interior, u(nv, ncells, ncells,
+ * [ncells]) one after another (amun_dev_upload_blocks and _download_blocks
+ * without the ghost layers).  On a multi-level mesh the blocks are in the
+ * order of its meta table. */
+int  amun_dev_upload_interiors(amun_ctx* ctx, const double* u);
+int  amun_dev_download_interiors(amun_ctx* ctx, double* u);
 int  amun_dev_download_global(amun_ctx* ctx, double* u, double* q);
 
 /* new_time_step (evolution.F90:379-493): cmax reduction over all interior
