@@ -12,7 +12,7 @@
 //
 // Local Jacobians: cons2prim and the limiters are written out by hand; the
 // face flux Jacobian comes from evaluating the solver templates of physics.h
-// on dual numbers (dual.h), NCH input columns per pass.
+// on dual numbers (dual.h), one input column per lane.
 //
 // Arrays are FP64 in the block-pool layout of the forward solver
 // ([block][variable][cell], lidx<8> bricks).  Included by amun_dev.hip.
@@ -21,8 +21,6 @@
 #include "dual.h"
 
 namespace amun_dev {
-
-constexpr int kAdjNch = 4;          // Jacobian columns per dual pass
 
 // cell of a thread: block b and (i, j, k) inside it
 __device__ __forceinline__ bool adj_cell(const RunConst& rc, int& b, int& i, int& j, int& k) {
@@ -34,6 +32,18 @@ __device__ __forceinline__ bool adj_cell(const RunConst& rc, int& b, int& i, int
   j = (c / nc) % nc;
   k = (rc.nd == 3) ? c / (nc * nc) : 0;
   return true;
+}
+
+// cell gid of the pool
+template <int ND>
+__device__ __forceinline__ void cell_of(const RunConst& rc, long long gid, int& b, int& i, int& j,
+                                        int& k) {
+  const int nc = rc.nc;
+  b = (int)(gid / rc.ncell);
+  const int c = (int)(gid - (long long)b * rc.ncell);
+  i = c % nc;
+  j = (c / nc) % nc;
+  k = ND == 3 ? c / (nc * nc) : 0;
 }
 
 template <int NV>
@@ -179,31 +189,14 @@ __device__ __forceinline__ double c2p_adjoint(const RunConst& rc, const double* 
 }
 
 // ---------------------------------------------------------------------------
-// face kernels: thread = cell i, face i+1/2 along DIR
+// face kernels: face i+1/2 along DIR of cell i
 // ---------------------------------------------------------------------------
-// face states of face i+1/2 (left from cell i, right from cell i+1)
-template <class P, int ND, int DIR>
-__device__ __forceinline__ void face_states(const double* __restrict__ Q, const int* __restrict__ nbr,
-                                            const RunConst& rc, int b, int i, int j, int k,
-                                            double* ql, double* qr) {
-#pragma unroll
-  for (int v = 0; v < P::nv; v++) {
-    double dm, d0, dp;
-    const double sl = slope_d<P, ND, DIR>(Q, nbr, rc, b, i, j, k, 0, v, dm, d0, dp);
-    const double sr = slope_d<P, ND, DIR>(Q, nbr, rc, b, i, j, k, 1, v, dm, d0, dp);
-    const double q0 = Q[var_index<P::nv>(rc, cell_index<8>(nbr, rc, b, i, j, k), v)];
-    const double q1 = Q[var_index<P::nv>(rc, cell_index<8>(nbr, rc, b, i + (DIR == 0), j + (DIR == 1), k + (DIR == 2)), v)];
-    ql[v] = q0 + sl;
-    qr[v] = q1 - sr;
-  }
-}
-
 // tangent of the face flux: DF(i) = dF(i+1/2) for tangent dX, dgamma
 // TF: arithmetic of the face flux and its Jacobian (double, or float in the
 // FP32-flux mode, whose forward evaluates the fluxes in float); everything
 // else -- primitives, slopes, the stage combines -- stays FP64
 template <class P, int RS, int ND, int DIR, typename TF>
-__global__ void k_tlm_face(const double* __restrict__ X, const double* __restrict__ Q,
+__global__ __launch_bounds__(256) void k_tlm_face(const double* __restrict__ X, const double* __restrict__ Q,
                            const double* __restrict__ dX, double dgam, double* __restrict__ DF,
                            const int* __restrict__ nbr, RunConst rc, double cmax) {
   int b, i, j, k;
@@ -254,63 +247,66 @@ __global__ void k_tlm_face(const double* __restrict__ X, const double* __restric
 
 // adjoint of the face flux: from MU (= c dt lambda_Y) the face flux adjoint
 // lF = dxi (MU(i+1) - MU(i)), then AL(i) = (dF/dqL)^T lF, AR(i) = (dF/dqR)^T
-// lF, GF(i) = (dF/dgamma) . lF
+// lF, GF(i) = (dF/dgamma) . lF.
+// A workgroup takes 64 faces: its waves form the face states and lF variable
+// by variable in LDS, then evaluate the Jacobian column by column, each lane
+// one face and one column (Dual<1>: about twice the solver's registers, two
+// waves per SIMD).  Bound by VALU issue.  One lane per face with four columns
+// at a time spilled 2 KB a lane and gave a 128^2 grid a quarter of the
+// chip's SIMDs: 595 us (x) and 637 us (y) a launch at 128^2 MHD HLLD, now
+// 54 and 49.
+constexpr int kAdjFaces = 64;
 template <class P, int RS, int ND, int DIR, typename TF>
-__global__ void k_adj_face(const double* __restrict__ Q, const double* __restrict__ MU,
-                           double* __restrict__ AL, double* __restrict__ AR,
-                           double* __restrict__ GF, const int* __restrict__ nbr, RunConst rc,
-                           double dxi, double cmax) {
-  int b, i, j, k;
-  if (!adj_cell(rc, b, i, j, k)) return;
+__global__ __launch_bounds__(256, 2) void k_adj_face(
+    const double* __restrict__ Q, const double* __restrict__ MU, double* __restrict__ AL,
+    double* __restrict__ AR, double* __restrict__ GF, const int* __restrict__ nbr, RunConst rc,
+    double dxi, double cmax) {
   constexpr int NV = P::nv;
-  double ql[NV], qr[NV], lf[NV];
-  face_states<P, ND, DIR>(Q, nbr, rc, b, i, j, k, ql, qr);
-  {
-    double m0[NV], m1[NV];
-    load_vec<NV>(MU, rc, cell_index<8>(nbr, rc, b, i, j, k), m0);
-    load_vec<NV>(MU, rc, cell_index<8>(nbr, rc, b, i + (DIR == 0), j + (DIR == 1), k + (DIR == 2)), m1);
-#pragma unroll
-    for (int v = 0; v < NV; v++) lf[v] = dxi * (m1[v] - m0[v]);
+  __shared__ double sl[NV][kAdjFaces], sr[NV][kAdjFaces], sf[NV][kAdjFaces];
+  const int f = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const long long gid = (long long)blockIdx.x * kAdjFaces + f;
+  const bool active = gid < (long long)rc.nblk * rc.ncell;
+  int b = 0, i = 0, j = 0, k = 0;
+  if (active) {
+    cell_of<ND>(rc, gid, b, i, j, k);
+    const size_t p0 = cell_index<8>(nbr, rc, b, i, j, k);
+    const size_t p1 =
+        cell_index<8>(nbr, rc, b, i + (DIR == 0), j + (DIR == 1), k + (DIR == 2));
+    for (int v = w; v < NV; v += 4) {
+      double dm, d0, dp;
+      const double l = slope_d<P, ND, DIR>(Q, nbr, rc, b, i, j, k, 0, v, dm, d0, dp);
+      const double r = slope_d<P, ND, DIR>(Q, nbr, rc, b, i, j, k, 1, v, dm, d0, dp);
+      sl[v][f] = Q[var_index<NV>(rc, p0, v)] + l;
+      sr[v][f] = Q[var_index<NV>(rc, p1, v)] - r;
+      sf[v][f] = dxi * (MU[var_index<NV>(rc, p1, v)] - MU[var_index<NV>(rc, p0, v)]);
+    }
   }
+  __syncthreads();
+  if (!active) return;
   // inputs in the solver's rotated frame: 0..NV-1 left, NV..2NV-1 right,
   // 2NV gamma
-  constexpr int NIN = 2 * NV + 1;
-  double gin[NIN];
-  for (int c0 = 0; c0 < NIN; c0 += kAdjNch) {
-    using DN = Dual<kAdjNch, TF>;
-    DN a[NV], c[NV], f[NV];
+  using D1 = Dual<1, TF>;
+  const size_t base = (size_t)b * NV * rc.ncell + lidx<8>(rc.nc, rc.nd, i, j, k);
+  for (int n = w; n <= 2 * NV; n += 4) {
+    D1 ql[NV], qr[NV], fl[NV];
 #pragma unroll
     for (int p = 0; p < NV; p++) {
-      a[p] = DN(ql[rot<P, DIR>(p)]);
-      c[p] = DN(qr[rot<P, DIR>(p)]);
+      ql[p] = D1(sl[rot<P, DIR>(p)][f]);
+      qr[p] = D1(sr[rot<P, DIR>(p)][f]);
+      ql[p].d[0] = TF(n == p ? 1 : 0);
+      qr[p].d[0] = TF(n == NV + p ? 1 : 0);
     }
-    DN g(rc.gamma);
+    D1 g(rc.gamma);
+    g.d[0] = TF(n == 2 * NV ? 1 : 0);
+    const EosConst<D1> e{g, g - 1.0, rcp(g - 1.0)};
+    riemann<P, RS, D1>(e, rc.sc, D1(cmax), D1(cmax * cmax), ql, qr, fl);
+    double acc = 0.0;
 #pragma unroll
-    for (int s = 0; s < kAdjNch; s++) {
-      const int n = c0 + s;
-      if (n < NV) a[n].d[s] = TF(1);
-      else if (n < 2 * NV) c[n - NV].d[s] = TF(1);
-      else if (n == 2 * NV) g.d[s] = TF(1);
-    }
-    const EosConst<DN> e{g, g - 1.0, rcp(g - 1.0)};
-    riemann<P, RS, DN>(e, rc.sc, DN(cmax), DN(cmax * cmax), a, c, f);
-#pragma unroll
-    for (int s = 0; s < kAdjNch; s++) {
-      const int n = c0 + s;
-      if (n >= NIN) break;
-      double acc = 0.0;
-#pragma unroll
-      for (int p = 0; p < NV; p++) acc += lf[rot<P, DIR>(p)] * double(f[p].d[s]);
-      gin[n] = acc;
-    }
+    for (int p = 0; p < NV; p++) acc += sf[rot<P, DIR>(p)][f] * double(fl[p].d[0]);
+    if (n < NV) AL[base + (size_t)rot<P, DIR>(n) * rc.ncell] = acc;
+    else if (n < 2 * NV) AR[base + (size_t)rot<P, DIR>(n - NV) * rc.ncell] = acc;
+    else GF[(size_t)b * rc.ncell + lidx<8>(rc.nc, rc.nd, i, j, k)] = acc;
   }
-  const size_t base = (size_t)b * NV * rc.ncell + lidx<8>(rc.nc, rc.nd, i, j, k);
-#pragma unroll
-  for (int p = 0; p < NV; p++) {
-    AL[base + (size_t)rot<P, DIR>(p) * rc.ncell] = gin[p];
-    AR[base + (size_t)rot<P, DIR>(p) * rc.ncell] = gin[NV + p];
-  }
-  GF[(size_t)b * rc.ncell + lidx<8>(rc.nc, rc.nd, i, j, k)] = gin[2 * NV];
 }
 
 // ---------------------------------------------------------------------------
@@ -347,23 +343,23 @@ __global__ void k_tlm_cell(const double* __restrict__ DF0, const double* __restr
 // cons2prim; LT(i) = (dL/dX)^T MU at i, GC(i) = the gamma part of the cell
 // (its cons2prim term plus the flux term of its upper faces)
 template <class P, int ND>
-__global__ void k_adj_cell(const double* __restrict__ X, const double* __restrict__ Q,
+__global__ __launch_bounds__(256) void k_adj_cell(const double* __restrict__ X, const double* __restrict__ Q,
                            const double* __restrict__ AL0, const double* __restrict__ AR0,
                            const double* __restrict__ AL1, const double* __restrict__ AR1,
                            const double* __restrict__ AL2, const double* __restrict__ AR2,
                            const double* __restrict__ GF0, const double* __restrict__ GF1,
                            const double* __restrict__ GF2, double* __restrict__ LT,
                            double* __restrict__ GC, const int* __restrict__ nbr, RunConst rc) {
-  int b, i, j, k;
-  if (!adj_cell(rc, b, i, j, k)) return;
   constexpr int NV = P::nv;
+  __shared__ double sq[NV][kAdjFaces];
+  const int f = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const long long gid = (long long)blockIdx.x * kAdjFaces + f;
+  const bool active = gid < (long long)rc.nblk * rc.ncell;
   const double* AL[3] = {AL0, AL1, AL2};
   const double* AR[3] = {AR0, AR1, AR2};
-  const size_t pc = cell_index<8>(nbr, rc, b, i, j, k);
-  double lq[NV];
-#pragma unroll
-  for (int v = 0; v < NV; v++) lq[v] = 0.0;
-  double gsum = 0.0;
+  int b = 0, i = 0, j = 0, k = 0, v = 0;
+  if (active) cell_of<ND>(rc, gid, b, i, j, k);
+  double lq = 0.0;
   auto per_dir = [&](auto dirc) {
     constexpr int D = decltype(dirc)::value;
     const int ei = (D == 0), ej = (D == 1), ek = (D == 2);
@@ -375,32 +371,40 @@ __global__ void k_adj_cell(const double* __restrict__ X, const double* __restric
       pcell[m] = cell_index<8>(nbr, rc, b, i + ei * o, j + ej * o, k + ek * o);
       pface[m] = cell_index<8>(nbr, rc, b, i + ei * (o - 1), j + ej * (o - 1), k + ek * (o - 1));
     }
-#pragma unroll
-    for (int v = 0; v < NV; v++) {
+    {
       // direct terms: qL(i+1/2) = q_i + s_i, qR(i-1/2) = q_i - s_i
-      lq[v] += AL[D][var_index<NV>(rc, pcell[1], v)] + AR[D][var_index<NV>(rc, pface[1], v)];
+      lq += AL[D][var_index<NV>(rc, pcell[1], v)] + AR[D][var_index<NV>(rc, pface[1], v)];
       double dm, d0, dp;
       // slope of cell i-1: d/dq_i is its "plus" partial
       slope_d<P, ND, D>(Q, nbr, rc, b, i, j, k, -1, v, dm, d0, dp);
-      lq[v] += (AL[D][var_index<NV>(rc, pcell[0], v)] - AR[D][var_index<NV>(rc, pface[0], v)]) * dp;
+      lq += (AL[D][var_index<NV>(rc, pcell[0], v)] - AR[D][var_index<NV>(rc, pface[0], v)]) * dp;
       slope_d<P, ND, D>(Q, nbr, rc, b, i, j, k, 0, v, dm, d0, dp);
-      lq[v] += (AL[D][var_index<NV>(rc, pcell[1], v)] - AR[D][var_index<NV>(rc, pface[1], v)]) * d0;
+      lq += (AL[D][var_index<NV>(rc, pcell[1], v)] - AR[D][var_index<NV>(rc, pface[1], v)]) * d0;
       slope_d<P, ND, D>(Q, nbr, rc, b, i, j, k, 1, v, dm, d0, dp);
-      lq[v] += (AL[D][var_index<NV>(rc, pcell[2], v)] - AR[D][var_index<NV>(rc, pface[2], v)]) * dm;
+      lq += (AL[D][var_index<NV>(rc, pcell[2], v)] - AR[D][var_index<NV>(rc, pface[2], v)]) * dm;
     }
   };
-  per_dir(std::integral_constant<int, 0>());
-  per_dir(std::integral_constant<int, 1>());
-  if constexpr (ND == 3) per_dir(std::integral_constant<int, 2>());
+  for (v = w; active && v < NV; v += 4) {
+    lq = 0.0;
+    per_dir(std::integral_constant<int, 0>());
+    per_dir(std::integral_constant<int, 1>());
+    if constexpr (ND == 3) per_dir(std::integral_constant<int, 2>());
+    sq[v][f] = lq;
+  }
+  __syncthreads();
+  if (!active || w) return;
+  const size_t pc = cell_index<8>(nbr, rc, b, i, j, k);
   const size_t pg = (size_t)b * rc.ncell + lidx<8>(rc.nc, rc.nd, i, j, k);
-  gsum += GF0[pg] + GF1[pg];
+  double gsum = GF0[pg] + GF1[pg];
   if constexpr (ND == 3) gsum += GF2[pg];
-  double u[NV], q[NV], lu[NV];
+  double u[NV], q[NV], lu[NV], ls[NV];
   load_vec<NV>(X, rc, pc, u);
   load_vec<NV>(Q, rc, pc, q);
-  gsum += c2p_adjoint<P>(rc, u, q, lq, lu);
 #pragma unroll
-  for (int v = 0; v < NV; v++) LT[var_index<NV>(rc, pc, v)] = lu[v];
+  for (int n = 0; n < NV; n++) ls[n] = sq[n][f];
+  gsum += c2p_adjoint<P>(rc, u, q, ls, lu);
+#pragma unroll
+  for (int n = 0; n < NV; n++) LT[var_index<NV>(rc, pc, n)] = lu[n];
   GC[pg] = gsum;
 }
 

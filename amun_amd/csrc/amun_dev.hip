@@ -2493,6 +2493,7 @@ int amun_dev_tape_backward(amun_ctx* c, const double* lam, double* lam0, double*
   if ((r = grad_state(c, keep, false))) return r;
   const long long nn = (long long)n;
   const dim3 gc((unsigned)(((long long)ncell + 255) / 256)), bl(256);
+  const dim3 gface((unsigned)((ncell + kAdjFaces - 1) / kAdjFaces));
   if ((r = global_to_pool(c, lam, B.LU0))) return r;     // lambda of U^N
   RunState h;
   HIP_TRY(hipMemcpy(&h, c->rs, sizeof(RunState), hipMemcpyDeviceToHost));
@@ -2516,10 +2517,10 @@ int amun_dev_tape_backward(amun_ctx* c, const double* lam, double* lam0, double*
                            0.0, B.MU);
         hipLaunchKernelGGL(d.adj_prim, gc, bl, 0, c->stream, X, B.Q, rc);
         for (int dd = 0; dd < nd; dd++)
-          hipLaunchKernelGGL(d.adj_face[dd], gc, bl, 0, c->stream, B.Q, B.MU, B.AL[dd], B.AR[dd],
+          hipLaunchKernelGGL(d.adj_face[dd], gface, bl, 0, c->stream, B.Q, B.MU, B.AL[dd], B.AR[dd],
                              B.GF[dd], c->nbr, rc, h.dxi[dd], T.cmax[s]);
         const int z = nd == 3 ? 2 : 1;
-        hipLaunchKernelGGL(d.adj_cell, gc, bl, 0, c->stream, X, B.Q, B.AL[0], B.AR[0], B.AL[1],
+        hipLaunchKernelGGL(d.adj_cell, gface, bl, 0, c->stream, X, B.Q, B.AL[0], B.AR[0], B.AL[1],
                            B.AR[1], B.AL[z], B.AR[z], B.GF[0], B.GF[1], B.GF[z], B.LT, B.GC,
                            c->nbr, rc);
         hipLaunchKernelGGL(k_sum_acc, dim3(npart), bl, 0, c->stream, B.GC, (long long)ncell, B.GP);
