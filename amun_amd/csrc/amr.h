@@ -248,44 +248,41 @@ __device__ __forceinline__ void face_flux(const RunConst& rc, const T* __restric
   for (int p = 0; p < NV; p++) f[rot<P, DIR>(p)] = fr[p];
 }
 
-// Averaged fine fluxes of the coarse faces with finer neighbours, one
-// thread per coarse face cell: x = correction slot, y = face cell of the
-// coarse block (c1 + nc c2), z = fine block, w = its lower-corner fine face
-// cell (f1 | f2 << 8) and face (0 or nc) << 16.  FB[slot][var][face cell].
+// Averaged fine fluxes of the coarse faces with finer neighbours, one lane
+// per fine face, the 2^(d-1) of a coarse face cell side by side: x =
+// correction slot, y = face cell of the coarse block (c1 + nc c2), z = fine
+// block, w = its lower-corner fine face cell (f1 | f2 << 8) and face (0 or
+// nc) << 16.  FB[slot][var][face cell].  Bound by latency (a few thousand
+// faces).  With all four solves in one lane the kernel spilled 1.5 KB a lane:
+// 104 us a direction on the 1576-leaf MHD mesh, now 21 us.
 template <class P, int REC, int RS, int ND, int DIR, typename T>
-static __global__ void k_amr_fineflux(const int4* __restrict__ task, int ntask, const void* Q,
-                                      const int* __restrict__ nbr, RunConst rc,
-                                      const RunState* __restrict__ rs, int slot,
-                                      double* __restrict__ FB, DevState* st,
-                                      const int* __restrict__ blev, const void* mlps_,
-                                      const void* mlpg_) {
-  constexpr int NV = P::nv;
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
+static __global__ __launch_bounds__(256, 2) void k_amr_fineflux(
+    const int4* __restrict__ task, int ntask, const void* Q, const int* __restrict__ nbr,
+    RunConst rc, const RunState* __restrict__ rs, int slot, double* __restrict__ FB, DevState* st,
+    const int* __restrict__ blev, const void* mlps_, const void* mlpg_) {
+  constexpr int NV = P::nv, kShare = ND == 3 ? 4 : 2;
+  const int g = blockIdx.x * blockDim.x + threadIdx.x, n = g / kShare, s = g % kShare;
+  // the lanes of one coarse face cell are all there or none is
   if (n >= ntask) return;
   const int4 t = task[n];
-  const int f1 = t.w & 0xff, f2 = (t.w >> 8) & 0xff, c = (t.w >> 16) & 0xff;
+  const int f1 = (t.w & 0xff) + (s & 1), f2 = ((t.w >> 8) & 0xff) + (s >> 1);
+  const int c = (t.w >> 16) & 0xff;
   const double cmaxd = cmax_of(rs, slot);
   const T cmax = T(cmaxd), cmax2 = T(cmaxd * cmaxd);
-  const T* Qp = static_cast<const T*>(Q);
-  const T* mlps = static_cast<const T*>(mlps_);
-  const T* mlpg = static_cast<const T*>(mlpg_);
-  T fa[NV], fb[NV];
+  T f[NV];
   const int nf = (ND == 3) ? rc.nc * rc.nc : rc.nc;
-  double* out = FB + (size_t)t.x * NV * nf + t.y;
   const double h = rs->h[DIR] / double(1 << blev[t.z]);   // the fine block's cell size
-  face_flux<P, REC, RS, ND, DIR, T>(rc, Qp, nbr, t.z, c, f1, f2, cmax, cmax2, st, h, mlps, mlpg, fa);
-  face_flux<P, REC, RS, ND, DIR, T>(rc, Qp, nbr, t.z, c, f1 + 1, f2, cmax, cmax2, st, h, mlps, mlpg, fb);
-  if constexpr (ND == 2) {
+  face_flux<P, REC, RS, ND, DIR, T>(rc, static_cast<const T*>(Q), nbr, t.z, c, f1, f2, cmax, cmax2,
+                                    st, h, static_cast<const T*>(mlps_),
+                                    static_cast<const T*>(mlpg_), f);
+  double* out = FB + (size_t)t.x * NV * nf + t.y;
 #pragma unroll
-    for (int v = 0; v < NV; v++) out[(size_t)v * nf] = (double(fa[v]) + double(fb[v])) / 2.0;
-  } else {
-    T fc[NV], fd[NV];
-    face_flux<P, REC, RS, ND, DIR, T>(rc, Qp, nbr, t.z, c, f1, f2 + 1, cmax, cmax2, st, h, mlps, mlpg, fc);
-    face_flux<P, REC, RS, ND, DIR, T>(rc, Qp, nbr, t.z, c, f1 + 1, f2 + 1, cmax, cmax2, st, h, mlps, mlpg, fd);
-    // ((l,l) + (p,p)) + ((l,p) + (p,l)) over the two transverse axes
-#pragma unroll
-    for (int v = 0; v < NV; v++)
-      out[(size_t)v * nf] = ((double(fa[v]) + double(fd[v])) + (double(fc[v]) + double(fb[v]))) / 4.0;
+  for (int v = 0; v < NV; v++) {
+    // 3D: ((l,l) + (p,p)) + ((l,p) + (p,l)) over the two transverse axes
+    double x = double(f[v]);
+    x = x + __shfl_xor(x, kShare - 1);
+    if constexpr (ND == 3) x = x + __shfl_xor(x, 1);
+    if (s == 0) out[(size_t)v * nf] = x / double(kShare);
   }
 }
 

@@ -1360,7 +1360,9 @@ static int amr_fill(amun_ctx* c, int qcur, int slot) {
   }
   for (int d = 0; d < c->rc.nd; d++)
     if (A.nf[d])
-      hipLaunchKernelGGL(c->disp.fineflux[d], dim3((A.nf[d] + 255) / 256), bl, 0, c->stream,
+      hipLaunchKernelGGL(c->disp.fineflux[d],
+                         dim3((unsigned)(((long long)A.nf[d] * (c->rc.nd == 3 ? 4 : 2) + 255) / 256)),
+                         bl, 0, c->stream,
                          A.ftask[d], A.nf[d], (const void*)c->Q[qcur], c->nbr, c->rc, c->rs,
                          slot, A.FB, A.dummy, (const int*)A.blev, (const void*)c->mlps,
                          (const void*)c->mlpg);
