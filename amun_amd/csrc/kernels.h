@@ -791,22 +791,35 @@ struct Recon<P, REC_TVD, ND, DIR, T> {
                                        const T* __restrict__ Q,
                                        const int* __restrict__ nbr, int b, int i, int j,
                                        int k, DevState* st, double) {
+    // density and pressure of the transverse neighbours: all loads first, on
+    // one address per neighbour (interleaved with the limiters, each its own
+    // index and wait: 467 instead of 385 us for the x sweep of 6.5 M cells)
+    T tm[2][3], tp[2][3];
+#pragma unroll
+    for (int d = 0; d < ND; d++) {
+      if (d == DIR) continue;
+      const size_t m = cell_index<sizeof(T)>(nbr, rc, b, i - (d == 0), j - (d == 1), k - (d == 2));
+      const size_t p = cell_index<sizeof(T)>(nbr, rc, b, i + (d == 0), j + (d == 1), k + (d == 2));
+      const T* __restrict__ Qm = Q + var_index<P::nv>(rc, m, P::idn);
+      const T* __restrict__ Qu = Q + var_index<P::nv>(rc, p, P::idn);
+      tm[0][d] = *Qm;
+      tp[0][d] = *Qu;
+      if constexpr (P::ipr >= 0) {
+        tm[1][d] = Qm[(P::ipr - P::idn) * rc.ncell];
+        tp[1][d] = Qu[(P::ipr - P::idn) * rc.ncell];
+      }
+    }
 #pragma unroll
     for (int v = 0; v < P::nv; v++) {
       const T qc = w[v][1];
       T dq = limiter<T>(rc.limiter, T(0.5), qc - w[v][0], w[v][2] - qc);
       if (v == P::idn || v == P::ipr) {
+        const int x = v == P::idn ? 0 : 1;
         T dqt[3] = {T(0), T(0), T(0)};
         dqt[DIR] = dq;
 #pragma unroll
-        for (int d = 0; d < ND; d++) {
-          if (d == DIR) continue;
-          int im = i - (d == 0), jm = j - (d == 1), km = k - (d == 2);
-          int ip = i + (d == 0), jp = j + (d == 1), kp = k + (d == 2);
-          T qm = Q[var_index<P::nv>(rc, cell_index<sizeof(T)>(nbr, rc, b, im, jm, km), v)];
-          T qp = Q[var_index<P::nv>(rc, cell_index<sizeof(T)>(nbr, rc, b, ip, jp, kp), v)];
-          dqt[d] = limiter<T>(rc.limiter, T(0.5), qc - qm, qp - qc);
-        }
+        for (int d = 0; d < ND; d++)
+          if (d != DIR) dqt[d] = limiter<T>(rc.limiter, T(0.5), qc - tm[x][d], tp[x][d] - qc);
         if (qc > T(0)) {
           // a finite slope falls below qc within kMaxHalvings halvings; the
           // bound only stops an infinite one (the reference loops forever)
