@@ -142,48 +142,40 @@ __device__ __forceinline__ T limiter(int kind, T x, T a, T b) {
 // ---------------------------------------------------------------------------
 // YC = true: reconstruct_weno5yc (interpolations.F90:2107-2254), whose tau
 // is the squared fourth difference (6 f(i) - 4 (f(i-1) + f(i+1)) + f(i-2) +
-// f(i+2))^2; everything else is WENO5-Z's
+// f(i+2))^2; everything else is WENO5-Z's.
+// The sweeps are bound by VALU issue and half of their operations stand here,
+// so the weights and interpolations are written for few of them (70 FP64 ones
+// per variable, the two reciprocals included, against 83 with the polynomials'
+// coefficients and the reference's scaling): smoothness indicators and eps
+// times 4, weights times 10 (both cancel in the quotient), and each
+// interpolation as the cell value plus a sum of first differences, which also
+// rounds relative to the differences and not to the value.
+// At 256^3 MHD: x sweep 1.07 -> 1.02 ms, y 1.09 -> 1.05; FP32 error of a
+// 48^3 run against 64 bits 4.2e-8 -> 3.5e-8.
 template <typename T, bool YC = false>
 __device__ __forceinline__ void weno5z_cell(const T f[5], T eps, T& fl, T& fr) {
-  const T c1 = T(13.0 / 12.0), c2 = T(0.25);
-  const T dl = T(0.1), dc = T(0.6), dr = T(0.3);
-  const T a11 = T(2.0 / 6.0), a12 = T(-7.0 / 6.0), a13 = T(11.0 / 6.0);
-  const T a21 = T(-1.0 / 6.0), a22 = T(5.0 / 6.0), a23 = T(2.0 / 6.0);
-  const T a31 = T(2.0 / 6.0), a32 = T(5.0 / 6.0), a33 = T(-1.0 / 6.0);
-  // dfm(i) = f(i)-f(i-1), dfp(i) = f(i+1)-f(i); df2(i) = c1*(dfp-dfm)^2
-  const T dfm_m1 = f[1] - f[0];
-  const T dfm_0 = f[2] - f[1];
-  const T dfp_0 = f[3] - f[2];
-  const T dfp_p1 = f[4] - f[3];
-  const T dfp_m1 = dfm_0, dfm_p1 = dfp_0;
-  T t;
-  t = dfp_m1 - dfm_m1; const T df2_m1 = c1 * (t * t);
-  t = dfp_0 - dfm_0;   const T df2_0 = c1 * (t * t);
-  t = dfp_p1 - dfm_p1; const T df2_p1 = c1 * (t * t);
-  t = T(3) * dfm_0 - dfm_m1; const T bl = df2_m1 + c2 * (t * t);
-  t = dfp_0 + dfm_0;         const T bc = df2_0 + c2 * (t * t);
-  t = T(3) * dfp_0 - dfp_p1; const T br = df2_p1 + c2 * (t * t);
+  const T c1 = T(13.0 / 3.0), sixth = T(1.0 / 6.0);
+  const T d0 = f[1] - f[0], d1 = f[2] - f[1], d2 = f[3] - f[2], d3 = f[4] - f[3];
+  const T s0 = d1 - d0, s1 = d2 - d1, s2 = d3 - d2;
+  const T ul = T(3) * d1 - d0, uc = d2 + d1, ur = T(3) * d2 - d3;
+  // 4 beta_k: 13/3 (second difference)^2 + (first difference)^2
+  const T bl = (c1 * s0) * s0 + ul * ul;
+  const T bc = (c1 * s1) * s1 + uc * uc;
+  const T br = (c1 * s2) * s2 + ur * ur;
   T tt;
   if constexpr (YC) {
-    const T d4 = (T(6) * f[2] - T(4) * (f[1] + f[3])) + (f[0] + f[4]);
-    tt = d4 * d4;
+    const T d4 = s2 - T(2) * s1 + s0;
+    tt = T(4) * (d4 * d4);
   } else {
     tt = tabs(br - bl);
   }
-  // the three interpolations of each face
-  const T ql = a11 * f[0] + a12 * f[1] + a13 * f[2];
-  const T qc = a21 * f[1] + a22 * f[2] + a23 * f[3];
-  const T qr = a31 * f[2] + a32 * f[3] + a33 * f[4];
-  const T pl = a11 * f[4] + a12 * f[3] + a13 * f[2];
-  const T pc = a21 * f[3] + a22 * f[2] + a23 * f[1];
-  const T pr = a31 * f[2] + a32 * f[1] + a33 * f[0];
   // alpha_k = 1 + tau/(beta_k + eps) (eq. 28 of Borges et al. 2008, p = 1);
-  // the normalised weights w_k = d_k alpha_k / sum(d alpha) are formed
-  // without the reference's three alpha divisions: in FP64 all alphas are
-  // scaled by (e_l e_c e_r), e_k = beta_k + eps, which leaves one division
-  // per face; in FP32 the alphas use the hardware reciprocal
+  // in FP64 all alphas are scaled by (e_l e_c e_r), e_k = 4 (beta_k + eps),
+  // which leaves one division per face; in FP32 they use the hardware
+  // reciprocal
   T gl, gc, gr;
-  const T el = bl + eps, ec = bc + eps, er = br + eps;
+  const T e4 = T(4) * eps;
+  const T el = bl + e4, ec = bc + e4, er = br + e4;
   if constexpr (sizeof(T) == 8) {
     gl = (el + tt) * (ec * er);
     gc = (ec + tt) * (el * er);
@@ -193,12 +185,14 @@ __device__ __forceinline__ void weno5z_cell(const T f[5], T eps, T& fl, T& fr) {
     gc = T(1) + tt * rcp(ec);
     gr = T(1) + tt * rcp(er);
   }
-  // left state of the upper face (weights dl, dc, dr on gl, gc, gr) and
-  // right state of the lower face (mirrored stencils, gl and gr swapped)
-  const T wl = dl * gl, wc = dc * gc, wr = dr * gr;
-  const T vl = dl * gr, vr = dr * gl;
-  fl = dv((wl * ql + wr * qr) + wc * qc, (wl + wr) + wc);
-  fr = dv((vl * pl + vr * pr) + wc * pc, (vl + vr) + wc);
+  // left state of the upper face (weights 1, 6, 3 on gl, gc, gr) and right
+  // state of the lower face (mirrored stencils, gl and gr swapped); the
+  // interpolations are f(i) plus or minus a sixth of these sums
+  const T wc = T(6) * gc, wr = T(3) * gr, vr = T(3) * gl;
+  const T ql = T(5) * d1 - T(2) * d0, qc = d1 + T(2) * d2, qr = T(4) * d2 - d3;
+  const T pl = T(5) * d2 - T(2) * d3, pc = d2 + T(2) * d1, pr = T(4) * d1 - d0;
+  fl = f[2] + sixth * dv((gl * ql + wr * qr) + wc * qc, (gl + wr) + wc);
+  fr = f[2] - sixth * dv((gr * pl + vr * pr) + wc * pc, (gr + vr) + wc);
 }
 
 // ---------------------------------------------------------------------------
