@@ -226,6 +226,7 @@ __device__ __forceinline__ void face_flux(const RunConst& rc, const T* __restric
   int i, j, k;
   const int pen = c1 + rc.nc * c2;
   coords(c - 1, i, j, k);
+  rec.prefetch(rc, Qp, nbr, b, i, j, k);
   rec.cell(rc, flm, frm, Qp, nbr, b, i, j, k, st, h);
   if (mlps)
     mlp_apply<P, ND, DIR, T>(rc, Qp, mlps, mlpg, nbr, b, c - 1, pen, i, j, k,
@@ -234,6 +235,7 @@ __device__ __forceinline__ void face_flux(const RunConst& rc, const T* __restric
   loadq(c + RC::R, qtmp);
   rec.load(2 * RC::R, qtmp);
   coords(c, i, j, k);
+  rec.prefetch(rc, Qp, nbr, b, i, j, k);
   rec.cell(rc, flc, frc, Qp, nbr, b, i, j, k, st, h);
   if (mlps)
     mlp_apply<P, ND, DIR, T>(rc, Qp, mlps, mlpg, nbr, b, c, pen, i, j, k, false, flc, frc);

@@ -402,7 +402,8 @@ SweepShape sweep_shape(const amun_ctx* c, int dir, int wg) {
     if ((long long)np * lanes(s.np) >= (long long)s.np * lanes(np)) s.np = np;
   s.lanes = lanes(s.np);
   s.grid = (unsigned)((total + s.np - 1) / s.np);
-  s.lds = sweep_lds_elems(c->nv, c->disp.R, rc.nc, s.np, dir) * c->qsize;
+  s.lds = sweep_lds_elems(c->nv, (int)c->qsize, relativistic(c->cfg), c->disp.R, rc.nc, s.np, dir) *
+          c->qsize;
   return s;
 }
 

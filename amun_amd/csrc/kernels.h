@@ -346,6 +346,8 @@ struct Recon;
 // WENO5-Z window of five cells (interfaces_dir -> reconstruct_weno5z)
 template <class P, int ND, int DIR, typename T>
 struct Recon<P, REC_WENO5Z, ND, DIR, T> {
+  __device__ __forceinline__ void prefetch(const RunConst&, const T*, const int*, int, int, int,
+                                           int) {}
   static constexpr int R = 2;    // window half width
   static constexpr int H = 3;    // ghost depth needed (faces of cells -1, nc)
   T w[P::nv][5];
@@ -404,6 +406,8 @@ struct Recon<P, REC_MP5, ND, DIR, T> : Recon<P, REC_WENO5Z, ND, DIR, T> {
 // MP7 (reconstruct_mp7): a seven-cell window
 template <class P, int ND, int DIR, typename T>
 struct Recon<P, REC_MP7, ND, DIR, T> {
+  __device__ __forceinline__ void prefetch(const RunConst&, const T*, const int*, int, int, int,
+                                           int) {}
   static constexpr int R = 3;
   static constexpr int H = 4;
   T w[P::nv][7];
@@ -442,6 +446,8 @@ struct Recon<P, REC_GP, ND, DIR, T> : Recon<P, REC_WENO5Z, ND, DIR, T> {
 // three-cell window; both weigh by the cell size h of the sweep direction
 template <class P, int ND, int DIR, typename T>
 struct Recon<P, REC_WENO3, ND, DIR, T> {
+  __device__ __forceinline__ void prefetch(const RunConst&, const T*, const int*, int, int, int,
+                                           int) {}
   static constexpr int R = 1;
   static constexpr int H = 2;
   T w[P::nv][3];
@@ -497,6 +503,8 @@ constexpr bool is_compact(int rec) {
 
 template <class P, int REC, int ND, int DIR, typename T>
 struct ReconCompact {
+  __device__ __forceinline__ void prefetch(const RunConst&, const T*, const int*, int, int, int,
+                                           int) {}
   static constexpr int R = 0;
   static constexpr int H = 2;
   __device__ __forceinline__ void load(int, const T*) {}
@@ -787,14 +795,14 @@ struct Recon<P, REC_TVD, ND, DIR, T> {
       w[v][1] = w[v][2];
     }
   }
-  __device__ __forceinline__ void cell(const RunConst& rc, T* flc, T* frc,
-                                       const T* __restrict__ Q,
-                                       const int* __restrict__ nbr, int b, int i, int j,
-                                       int k, DevState* st, double) {
-    // density and pressure of the transverse neighbours: all loads first, on
-    // one address per neighbour (interleaved with the limiters, each its own
-    // index and wait: 467 instead of 385 us for the x sweep of 6.5 M cells)
-    T tm[2][3], tp[2][3];
+  // density and pressure of the transverse neighbours
+  T tm[2][3], tp[2][3];
+  __device__ __forceinline__ void prefetch(const RunConst& rc, const T* __restrict__ Q,
+                                           const int* __restrict__ nbr, int b, int i, int j,
+                                           int k) {
+    // one address per neighbour, all loads before any use (interleaved with
+    // the limiters, each its own index and wait: 467 instead of 385 us for the
+    // x sweep of 6.5 M cells)
 #pragma unroll
     for (int d = 0; d < ND; d++) {
       if (d == DIR) continue;
@@ -809,6 +817,11 @@ struct Recon<P, REC_TVD, ND, DIR, T> {
         tp[1][d] = Qu[(P::ipr - P::idn) * rc.ncell];
       }
     }
+  }
+  __device__ __forceinline__ void cell(const RunConst& rc, T* flc, T* frc,
+                                       const T* __restrict__ Q,
+                                       const int* __restrict__ nbr, int b, int i, int j,
+                                       int k, DevState* st, double) {
 #pragma unroll
     for (int v = 0; v < P::nv; v++) {
       const T qc = w[v][1];
@@ -850,6 +863,8 @@ struct Recon<P, REC_TVD, ND, DIR, T> {
 // pair.
 template <class P, int ND, int DIR, typename T>
 struct Recon<P, REC_MGP, ND, DIR, T> {
+  __device__ __forceinline__ void prefetch(const RunConst&, const T*, const int*, int, int, int,
+                                           int) {}
   static constexpr int R = 0;
   static constexpr int H = 2;
   __device__ __forceinline__ void load(int, const T*) {}
@@ -1096,9 +1111,18 @@ __host__ __device__ constexpr int tile_width(int nc, int R, int dir) {
   return row_width(nc + 2 * (R + 1), dir);
 }
 __host__ __device__ constexpr int face_width(int nc, int dir) { return row_width(nc + 1, dir); }
-__host__ __device__ constexpr size_t sweep_lds_elems(int nv, int R, int nc, int np, int dir) {
+// whether the solver leaves registers for the cell's increment and states;
+// where not, the increment of the directions before waits in LDS
+__host__ __device__ constexpr bool sweep_loads_early(int nv, int es, bool sr) {
+  return nv * es <= 40 && !sr;
+}
+__host__ __device__ constexpr bool sweep_inc_lds(int nv, int es, bool sr, int R, int dir) {
+  return R > 0 && dir > 0 && !sweep_loads_early(nv, es, sr);
+}
+__host__ __device__ constexpr size_t sweep_lds_elems(int nv, int es, bool sr, int R, int nc,
+                                                     int np, int dir) {
   const int w = R ? tile_width(nc, R, dir) : face_width(nc, dir);
-  return (size_t)nv * np * w;
+  return (size_t)nv * np * (w + (sweep_inc_lds(nv, es, sr, R, dir) ? nc : 0));
 }
 
 // n / d for 0 <= n < 2^16, d > 0, with rd = 1 / d (exact: the distance of
@@ -1134,6 +1158,8 @@ __device__ __forceinline__ double sweep_cells(const SweepArgs& a, const RunConst
   constexpr bool kPair = sizeof(T) == 4 && ND == 3;   // bricks of two z planes (lidx)
   using RC = Recon<P, REC, ND, DIR, T>;
   constexpr int R = RC::R;
+  constexpr bool kEarly = sweep_loads_early(NV, sizeof(T), P::sr);
+  constexpr bool kIncLds = sweep_inc_lds(NV, sizeof(T), P::sr, R, DIR);
   const int nc = rc.nc, npen = (ND == 3) ? nc * nc : nc;
   const int wt = tile_width(nc, R, DIR), wf = face_width(nc, DIR), nf = np * wf;
   T* const face = smem;   // [var][pencil][cell + 1] upper states, [var][pencil][cell] fluxes
@@ -1219,41 +1245,106 @@ __device__ __forceinline__ double sweep_cells(const SweepArgs& a, const RunConst
   const unsigned ot = inner ? ob + lidx<sizeof(T)>(nc, ND, ci, cj, ck) : 0u;
   const size_t base0 = (size_t)b0 * nbk;
 
-  if constexpr (R > 0) {
-    if (inner) {
-      const T* __restrict__ Q0 = Qp + base0;
-#pragma unroll
-      for (int v = 0; v < NV; v++) smem[(v * np + p) * wt + c + R + 1] = at_byte(Q0 + v * rc.ncell, ot * (unsigned)sizeof(T));
-    }
-    // the R + 1 cells beyond each end
-    constexpr int H = 2 * (R + 1);
-    for (int x = lane; x < np * H; x += blockDim.x) {
-      const int ph = x / H, m = x - ph * H, ch = m <= R ? m - 1 - R : nc + m - 1 - R;
-      int hb, h1, h2, i, j, k;
-      pencil(ph, hb, h1, h2);
-      if (hb < rc.nblk) {
-        coords(ch, h1, h2, i, j, k);
-        const size_t pk = cell_index<sizeof(T)>(a.nbr, rc, hb, i, j, k);
-        const T* __restrict__ Qh = Qp + ((pk >> 32) * nbk + (pk & 0xffffffffull));
-#pragma unroll
-        for (int v = 0; v < NV; v++) smem[(v * np + ph) * wt + ch + R + 1] = Qh[v * rc.ncell];
-      }
-    }
-    __syncthreads();
-  }
-
+  // the loads that others wait for first: the run's state, the reconstruction's
+  // own neighbours, then the tile
   run = a.brun[b < rc.nblk ? b : b0];   // lanes without a cell: the first block's
   const RunState* Rs = a.rs + run;
   const double cmaxd = cmax_of(Rs, a.slot);
   const T cmax = T(cmaxd), cmax2 = T(cmaxd * cmaxd);
   const EosConst<T> e{T(rc.gamma), T(rc.gammam1), T(rc.gammam1i), T(rc.csnd), T(rc.csnd2)};
   double smax = 0.0;
+  RC rec;
+  if (active) rec.prefetch(rc, Qp, a.nbr, b, ci, cj, ck);
+
+  // All loads of the tile are issued before the first wait: the block across
+  // each end, the lane's own cell (and its increment, where the solver leaves
+  // no registers to load it later and ahead of its use), the cells beyond the
+  // ends.
+  T* __restrict__ Dp = static_cast<T*>(a.D) + base0;
+  T* const inc = smem + NV * np * (R ? wt : wf);   // [var][lane], kIncLds
+  constexpr int H = 2 * (R + 1);
+  if constexpr (R > 0) {
+    constexpr int kStep = DIR == 0 ? 1 : (DIR == 1 ? 3 : 9);
+    // the cells beyond the ends: m < H / 2 before cell 0, the others from nc on
+    auto halo = [&](int x, int& slot, const T*& from) {
+      const int ph = x / H, m = x - ph * H;
+      const bool low = m < H / 2;
+      int hb, h1, h2, i, j, k;
+      pencil(ph, hb, h1, h2);
+      if (hb >= rc.nblk) return false;
+      const int nb = a.nbr[hb * 27 + (low ? 13 - kStep : 13 + kStep)];
+      coords(low ? nc + m - H / 2 : m - H / 2, h1, h2, i, j, k);
+      from = Qp + ((size_t)nb * nbk + lidx<sizeof(T)>(nc, ND, i, j, k));
+      slot = ph * wt + (low ? m : nc + m);
+      return true;
+    };
+    int slot = 0;
+    const T* from = nullptr;
+    const bool has = lane < np * H && halo(lane, slot, from);
+    T q[NV], d[NV], h[NV];
+    if (inner) {
+      const T* __restrict__ Q0 = Qp + base0;
+#pragma unroll
+      for (int v = 0; v < NV; v++) q[v] = at_byte(Q0 + v * rc.ncell, ot * (unsigned)sizeof(T));
+      if constexpr (kIncLds) {
+#pragma unroll
+        for (int v = 0; v < NV; v++) d[v] = at_byte(Dp + v * rc.ncell, ot * (unsigned)sizeof(T));
+      }
+    }
+    if (has) {
+#pragma unroll
+      for (int v = 0; v < NV; v++) h[v] = from[v * rc.ncell];
+    }
+    if (inner) {
+#pragma unroll
+      for (int v = 0; v < NV; v++) smem[(v * np + p) * wt + c + R + 1] = q[v];
+      if constexpr (kIncLds) {
+#pragma unroll
+        for (int v = 0; v < NV; v++) inc[v * nin + lane] = d[v];
+      }
+    }
+    if (has) {
+#pragma unroll
+      for (int v = 0; v < NV; v++) smem[v * np * wt + slot] = h[v];
+    }
+    for (int x = lane + blockDim.x; x < np * H; x += blockDim.x)   // blocks of 4 cells
+      if (halo(x, slot, from))
+#pragma unroll
+        for (int v = 0; v < NV; v++) smem[v * np * wt + slot] = from[v * rc.ncell];
+    __syncthreads();
+  }
+
+  // the cell's increment and states.  Where the solver leaves registers for
+  // them (kEarly), they are loaded before it, so that it covers their latency
+  const unsigned od = ob + lidx<8>(nc, ND, ci, cj, ck), of = ob + lidx<4>(nc, ND, ci, cj, ck);
+  T* __restrict__ Qo = static_cast<T*>(a.Qout) + base0;
+  double* Uo = a.Uout + base0;
+  float* Cp = sizeof(T) == 4 ? a.C + base0 : nullptr;
+  T dpre[NV];
+  double u0pre[NV], u1pre[NV];
+  float cpre[NV];
+  auto load_cell = [&]() {
+    const double* U0 = a.U0 + base0;
+    const double* U1 = a.U1 + base0;
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      const int off = v * rc.ncell;
+      if constexpr (kIncLds) dpre[v] = inc[v * nin + lane];
+      else if constexpr (DIR > 0) dpre[v] = at_byte(Dp + off, ot * (unsigned)sizeof(T));
+      if constexpr (kLast) {
+        u0pre[v] = at_byte(U0 + off, od * 8u);
+        u1pre[v] = a.kind != 0 ? at_byte(U1 + off, od * 8u) : 0.0;
+        // the compensation enters the updates of the step state; the
+        // transient stages ignore it (it is below the FP64 rounding of U0)
+        if constexpr (sizeof(T) == 4) cpre[v] = a.comp ? at_byte(Cp + off, of * 4u) : 0.0f;
+      }
+    }
+  };
 
   T flc[NV], frc[NV], f[NV];
   if (active) {
     // cell size along DIR at this block's level (coordinates.F90:330-341)
     const double hdir = a.blev ? Rs->h[DIR] / double(1 << a.blev[b]) : Rs->h[DIR];
-    RC rec;
     if constexpr (R > 0) {
 #pragma unroll
       for (int v = 0; v < NV; v++)
@@ -1284,6 +1375,9 @@ __device__ __forceinline__ double sweep_cells(const SweepArgs& a, const RunConst
     for (int v = 0; v < NV; v++) ql[v] = face[rot<P, DIR>(v) * nf + p * wf + c];
   }
   __syncthreads();   // the fluxes replace the face states
+  if constexpr (kEarly) {
+    if (inner) load_cell();
+  }
   if (active && c >= 0) {
     // face c-1/2: left state from cell c-1, right state from cell c
     T qr[NV], fr[NV];
@@ -1307,30 +1401,11 @@ __device__ __forceinline__ double sweep_cells(const SweepArgs& a, const RunConst
   }
   __syncthreads();
   if (inner) {
-    const unsigned od = ob + lidx<8>(nc, ND, ci, cj, ck), of = ob + lidx<4>(nc, ND, ci, cj, ck);
+    if constexpr (!kEarly) load_cell();
     const unsigned oc = ot - ob;      // the cell inside its block
-    T* __restrict__ Dp = static_cast<T*>(a.D) + base0;
-    T* __restrict__ Qo = static_cast<T*>(a.Qout) + base0;
-    const double* U0 = a.U0 + base0;
-    const double* U1 = a.U1 + base0;
-    double* Uo = a.Uout + base0;
-    float* Cp = sizeof(T) == 4 ? a.C + base0 : nullptr;
-    T dpre[NV], fn[NV];
-    double u0pre[NV], u1pre[NV];
-    float cpre[NV];
+    T fn[NV];
 #pragma unroll
-    for (int v = 0; v < NV; v++) {
-      const int off = v * rc.ncell;
-      if constexpr (DIR > 0) dpre[v] = at_byte(Dp + off, ot * (unsigned)sizeof(T));
-      if constexpr (kLast) {
-        u0pre[v] = at_byte(U0 + off, od * 8u);
-        if (a.kind != 0) u1pre[v] = at_byte(U1 + off, od * 8u);
-        // the compensation enters the updates of the step state; the
-        // transient stages ignore it (it is below the FP64 rounding of U0)
-        if constexpr (sizeof(T) == 4) cpre[v] = a.comp ? at_byte(Cp + off, of * 4u) : 0.0f;
-      }
-      fn[v] = face[v * nf + p * wf + c + 1];
-    }
+    for (int v = 0; v < NV; v++) fn[v] = face[v * nf + p * wf + c + 1];
     const double ds = kLast ? a.fac * dt_of(rc, Rs, a.slot, a.dtnext) : 0.0;
     const EosConst<double> ed{rc.gamma, rc.gammam1, rc.gammam1i, rc.csnd, rc.csnd2};
     const T dxi = T(a.blev ? Rs->dxi[DIR] * double(1 << a.blev[b]) : Rs->dxi[DIR]);
