@@ -392,6 +392,8 @@ struct SweepShape {
   size_t lds;
 };
 
+constexpr unsigned kComputeUnits = 256;
+
 SweepShape sweep_shape(const amun_ctx* c, int dir, int wg) {
   const RunConst& rc = c->rc;
   const long long total = (long long)rc.nblk * (rc.nd == 3 ? rc.nc * rc.nc : rc.nc);
@@ -1519,7 +1521,10 @@ static int enqueue_step(amun_ctx* c, double dtnext, int slot, int qcur, hipEvent
                            c->st);
       }
       a.swz = c->swz[dir];
-      const SweepShape w = sweep_shape(c, dir, c->wg[dir]);
+      SweepShape w = sweep_shape(c, dir, c->wg[dir]);
+      // a grid that leaves CUs idle: smaller workgroups on more of them (128^2
+      // HD, 74 workgroups of 14 pencils: 42.4 us a step, 171 of 6: 39.7)
+      if (w.grid < kComputeUnits) w = sweep_shape(c, dir, 128);
       a.np = w.np;
       hipLaunchKernelGGL(d.sweep[dir], dim3(w.grid), dim3(w.lanes), w.lds, c->stream, a, rc);
       parts = (int)w.grid;
@@ -1531,7 +1536,7 @@ static int enqueue_step(amun_ctx* c, double dtnext, int slot, int qcur, hipEvent
       HIP_TRY(hipMemcpyAsync(rec + (s + 1) * c->nstate, stages[s].to_u0 ? c->U0 : c->U1,
                              c->nstate * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
   }
-  hipLaunchKernelGGL(k_end_step, dim3((unsigned)std::max(1, std::min(64, parts / 1024))),
+  hipLaunchKernelGGL(k_end_step, dim3((unsigned)std::max(1, std::min(64, parts / 256))),
                      dim3(64 * kEndWaves), 0, c->stream, c->spart, parts, c->rs, c->trace,
                      c->tsteps, rc, slot, dtnext);
   if (ev) HIP_TRY(hipEventRecord(*ev++, c->stream));
@@ -2559,14 +2564,15 @@ int amun_dev_tape_backward(amun_ctx* c, const double* lam, double* lam0, double*
 }  // extern "C"
 
 // ---------------------------------------------------------------------------
-// the allocation-free cons2prim: its event counters live in a static device
-// array instead of a hipMalloc'd DevState
+// the allocation-free cons2prim.  A few thousand states take no longer than
+// the launches: clearing, recovery and a copy of static counters were three,
+// 12.6 us a call on 2000 SRMHD states; now @@C2P@@ (one launch for HD and MHD).
 // ---------------------------------------------------------------------------
 namespace {
 constexpr int kScratchWords = 32;   // 256 bytes: one DevState and room to spare
 static_assert(sizeof(DevState) <= kScratchWords * sizeof(unsigned long long),
               "DevState must fit the static scratch array");
-static __device__ __align__(256) unsigned long long scratch[kScratchWords];
+static __device__ __align__(256) unsigned long long scratch[kScratchWords];   // unread counts
 
 // device address of scratch on every device the library has run on (the
 // array's host-side name is not a device address)
@@ -2587,14 +2593,8 @@ int scratch_of_current_device(void** out) {
   return 0;
 }
 
-__global__ void k_scratch_clear(unsigned long long* p, int n) {
-  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (i < n) p[i] = 0ull;
-}
-
-__global__ void k_scratch_events(const DevState* st, int64_t* out) {
-  const int i = (int)threadIdx.x;
-  if (i < 3) out[i] = (int64_t)st->c2p[i];
+__global__ void k_clear_events(int64_t* p) {
+  if (threadIdx.x < 3) p[threadIdx.x] = 0;
 }
 }  // namespace
 
@@ -2608,17 +2608,23 @@ extern "C" int amun_dev_cons2prim_noalloc(const amun_cfg* cfg, int32_t n, const 
   Dispatch d;
   if (!pick(d, *cfg)) return fail(600, "no kernel instantiation for this configuration");
   const RunConst rc = make_rc(*cfg);
-  void* sp = nullptr;
-  r = scratch_of_current_device(&sp);
-  if (r) return r;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  unsigned long long* words = static_cast<unsigned long long*>(sp);
-  hipLaunchKernelGGL(k_scratch_clear, dim3(1), dim3(kScratchWords), 0, s, words, kScratchWords);
-  hipLaunchKernelGGL(d.unit_c2p, dim3((unsigned)((n + 127) / 128)), dim3(128), 0, s, n, d_u, d_q,
-                     rc, static_cast<DevState*>(sp));
-  if (d_events)
-    hipLaunchKernelGGL(k_scratch_events, dim3(1), dim3(64), 0, s,
-                       static_cast<const DevState*>(sp), d_events);
+  // the counts go straight into the caller's array (the kernel uses nothing
+  // of a DevState but c2p), without one to the static array, unread; only the
+  // relativistic recovery adds to them, the others' kernel clears them itself
+  DevState* st = nullptr;
+  if (d_events) {
+    st = reinterpret_cast<DevState*>(reinterpret_cast<char*>(d_events) - offsetof(DevState, c2p));
+    if (relativistic(*cfg))
+      hipLaunchKernelGGL(k_clear_events, dim3(1), dim3(64), 0, s, d_events);
+  } else {
+    void* sp = nullptr;
+    r = scratch_of_current_device(&sp);
+    if (r) return r;
+    st = static_cast<DevState*>(sp);
+  }
+  hipLaunchKernelGGL(d.unit_c2p, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, s, n, d_u, d_q, rc,
+                     st);
   HIP_TRY(hipGetLastError());
   return 0;
 }

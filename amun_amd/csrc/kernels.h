@@ -1945,6 +1945,8 @@ __global__ void k_unit_c2p(int n, const double* __restrict__ u, double* __restri
   } else {
     const EosConst<double> ed{rc.gamma, rc.gammam1, rc.gammam1i, rc.csnd, rc.csnd2};
     cons2prim<P, double>(ed, ud, qd);
+    if (i < 3) st->c2p[i] = 0;   // this recovery counts nothing
+    if (n < 3 && i == 0) st->c2p[1] = st->c2p[2] = 0;
   }
 #pragma unroll
   for (int v = 0; v < NV; v++) q[(size_t)i * NV + v] = qd[v];
