@@ -1111,8 +1111,11 @@ __host__ __device__ constexpr int tile_width(int nc, int R, int dir) {
   return row_width(nc + 2 * (R + 1), dir);
 }
 __host__ __device__ constexpr int face_width(int nc, int dir) { return row_width(nc + 1, dir); }
-// whether the solver leaves registers for the cell's increment and states;
-// where not, the increment of the directions before waits in LDS
+// Whether the solver leaves registers for the cell's increment and states
+// (HD, and every FP32 system but the relativistic: at most 10 words a state);
+// where not, the increment of the directions before waits in LDS: read at the
+// update instead, it cost 0.5 ms of a 256^3 FP64 MHD step, and early in
+// registers it spilled.
 __host__ __device__ constexpr bool sweep_loads_early(int nv, int es, bool sr) {
   return nv * es <= 40 && !sr;
 }
@@ -1147,8 +1150,18 @@ __device__ __forceinline__ X& at_byte(X* x, unsigned o) {
 // the 4-cell bricks, so that every access of a wave to its own cells is whole
 // 128-byte lines: with a pencil's cells on consecutive lanes instead, the z
 // sweep of the 128^3 MHD run sent 14.2 M write requests to L2 for 4.7 M full
-// ones and took 2.4 ms at 256^3.  Every thread of the workgroup must call
-// this.  Returns the maximum speed of the lane's new state (last sweep of a
+// ones and took 2.4 ms at 256^3.
+// The order of the loads: all of the tile's before the first wait, so that
+// the own cell does not wait while the neighbour look-up of the halo begins
+// (kEarly: the states and the increment too, which a solver of 40 bytes a cell
+// leaves registers for; where it does not, the increment waits in LDS).
+// 256^3 MHD WENO5-Z + HLLD: FP64 11.55 -> 11.07 ms a step, mixed 8.08 -> 7.56.
+// What bounds it: x and y vector issue and latency (0.99 and 1.0 ms a launch
+// at 256^3 in FP64; 1.29 and 1.59 with a pencil a lane), z the bytes of the
+// state, its stages and the increment (1.75 ms, 4.2 TB/s, where a device copy
+// reaches 5.0).  With a pencil a lane a grid of few cells left most SIMDs idle:
+// 128^2 HD TVD 281 -> 40 us a step, 340^2 MHD 707 -> 98, 512^2 SRMHD stages
+// 1168 -> 224.  Every thread of the workgroup must call this.  Returns the maximum speed of the lane's new state (last sweep of a
 // step).
 template <class P, int REC, int RS, int ND, int DIR, typename T>
 __device__ __forceinline__ double sweep_cells(const SweepArgs& a, const RunConst& rc, int g0,

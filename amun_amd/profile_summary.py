@@ -103,7 +103,7 @@ def main():
     wc, _ = counters(a.write)
     vc, vres = counters(a.valu)
     res.update(vres)
-    sweeps = sorted(k for k in st if "k_sweep" in k or "k_stage" in k)
+    sweeps = sorted(k for k in st if "k_sweep" in k)
     lines = [f"# rocprofv3 summary: 3D MHD-GLM WENO5-Z+HLLD SSPRK(3,3), {a.size}^3 "
              f"({cells // 4096} blocks of 16^3), precision {a.precision}"]
     lines += ["# " + c for c in a.commands.split("\n") if c.strip()]
@@ -142,8 +142,7 @@ def main():
         lines.append(f"  {k[:62]:62s} fp64 {a64:7.2f} GFLOP  fp32 {a32:7.2f} GFLOP  "
                      f"VALU-active/wave-cycles {act / cyc if cyc else 0:5.2f}  "
                      f"wait-any/wave-cycles {wait / cyc if cyc else 0:5.2f}")
-    # a step is three stages of one launch per direction (k_sweep) or one
-    # launch each (k_stage)
+    # a step is three stages of one launch per direction
     nst = 3
     step_us = sum(st[k][1] for k in sweeps) * nst
     step_bytes = (rd + wr) * 1e9 * nst

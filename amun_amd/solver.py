@@ -246,9 +246,8 @@ class Solver:
         self._check(self.lib.amun_dev_set_graph(self.h, int(enable)))
 
     def set_stage_fusion(self, enable: bool = True):
-        """One launch per stage: the x, y (and z) sweeps of a stage in one
-        kernel whose workgroups hold whole blocks (bitwise the same
-        results)."""
+        """Time a stage as a whole (timed_run) instead of every sweep of it;
+        the launches and the results are the same."""
         self._check(self.lib.amun_dev_set_stage_fusion(self.h, int(enable)))
 
     def autotune(self, nsteps: int = 3):

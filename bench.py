@@ -166,9 +166,9 @@ def main():
     ap.add_argument("--no-mixed", action="store_true",
                     help="skip the mixed-precision leg reported beside the FP64 value")
     ap.add_argument("--launch", default="fused", choices=["fused", "split"],
-                    help="one launch per stage (x, y, z sweeps in one kernel, "
-                         "amun_dev_set_stage_fusion) or one launch per sweep direction; "
-                         "the other is reported beside the value")
+                    help="with amun_dev_set_stage_fusion (timings per stage) or without "
+                         "(timings per sweep); the launches are the same; the other is "
+                         "reported beside the value")
     ap.add_argument("--no-other-launch", action="store_true",
                     help="skip the FP64 leg of the other launch mode")
     ap.add_argument("--no-cpu-baseline", action="store_true")
@@ -282,9 +282,7 @@ def main():
         roofline = {"bound": "valu", "achieved": valu["achieved"], "peak": valu["peak"],
                     "unit": valu["unit"], "frac": valu["frac"], "hbm": hbm}
     roofline.update({"traffic": traffic,
-                     "kernel": ("one SSPRK(3,3) step = 3 k_stage launches + k_end_step"
-                                if args.launch == "fused" else
-                                "one SSPRK(3,3) step = 9 k_sweep launches + k_end_step"),
+                     "kernel": "one SSPRK(3,3) step = 9 k_sweep launches + k_end_step",
                      "bytes_per_zone_update": bpz,
                      "device_ms_per_step": step_ms,
                      "kernel_ms_per_step": [round(float(x), 4) for x in kms]})

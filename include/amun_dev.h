@@ -272,20 +272,19 @@ int  amun_dev_statistics_run(amun_ctx* ctx, int32_t r, double out[21]);
 int  amun_dev_set_graph(amun_ctx* ctx, int32_t enable);
 
 /* Launch-shape autotuner: runs nsteps timed steps of the live state for every
- * candidate shape (workgroup of 64, 128 or 256 pencils; plain or XCD-grouped
+ * candidate shape (workgroup of 64, 128 or 256 lanes; plain or XCD-grouped
  * workgroup order), keeps the fastest per sweep direction and restores the
  * state, so the run continues as if the call had not happened.  choice (may
  * be NULL) receives ndims pairs (workgroup size, XCD grouping).
  * amun_dev_set_launch sets such pairs directly. */
 int  amun_dev_autotune(amun_ctx* ctx, int32_t nsteps, int32_t* choice);
 
-/* One launch per stage (no reference counterpart; the reference's evolve_*
- * calls update_fluxes once per stage, evolution.F90:628-1208): with
- * enable != 0 every stage runs its x, y (and z) sweeps in one kernel whose
- * workgroups hold whole blocks, with a workgroup barrier between the
- * directions.  For the TVD and WENO5-Z reconstructions of the HD and MHD
- * systems when ncells^(ndims-1) divides 256 (600 otherwise); the results
- * are bitwise those of the per-direction launches. */
+/* Per-stage timing (no reference counterpart; the reference's evolve_* calls
+ * update_fluxes once per stage, evolution.F90:628-1208): with enable != 0
+ * amun_dev_timed_run times every stage as a whole instead of every sweep of
+ * it.  The launches are the same: a sweep a direction, which is faster than
+ * one kernel a stage.  Accepted for the TVD and WENO5-Z reconstructions of the
+ * HD and MHD systems when ncells^(ndims-1) divides 256 (600 otherwise). */
 int  amun_dev_set_stage_fusion(amun_ctx* ctx, int32_t enable);
 int  amun_dev_set_launch(amun_ctx* ctx, const int32_t* choice);
 
