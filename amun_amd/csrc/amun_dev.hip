@@ -10,10 +10,40 @@
 
 #include <array>
 #include <map>
+#include <thread>
 
 // ===========================================================================
 // context
 // ===========================================================================
+// Pinned buffers of large downloads (copy_to_host), from the first of them to
+// the end of the context: two pieces a thread, each with the event of its copy
+constexpr int kStagedThreads = 4;
+constexpr size_t kStagedBytes = (size_t)64 << 20, kStagedPiece = (size_t)2 << 20;
+struct Staging {
+  char* pin = nullptr;
+  hipEvent_t done[2 * kStagedThreads] = {};
+  bool make() {
+    if (pin) return true;
+    bool ok = hipHostMalloc((void**)&pin, 2 * kStagedThreads * kStagedPiece,
+                            hipHostMallocDefault) == hipSuccess;
+    for (hipEvent_t& e : done)
+      ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    if (!ok) {
+      (void)hipGetLastError();
+      drop();
+    }
+    return ok;
+  }
+  void drop() {
+    if (pin) (void)hipHostFree(pin);
+    pin = nullptr;
+    for (hipEvent_t& e : done) {
+      if (e) (void)hipEventDestroy(e);
+      e = nullptr;
+    }
+  }
+};
+
 struct amun_ctx {
   amun_cfg cfg;
   RunConst rc;
@@ -37,7 +67,7 @@ struct amun_ctx {
   void* vsrc = nullptr;        // viscous and resistive source products per stage
   void* q4 = nullptr;          // four-velocity states of the stage input (relativistic)
   int vis = 0;                 // 1 viscosity, 2 resistivity (SweepArgs::vis)
-  int fuse = 0;                // one k_stage launch per stage (amun_dev_set_stage_fusion)
+  int fuse = 0;                // one timing event per stage (amun_dev_set_stage_fusion)
   void* mlps = nullptr;        // multi-dimensional limiting: slopes of the interior cells
   void* mlpg = nullptr;        // and of the cells beyond the pencil ends (k_mlp)
   int qcur = 0;                // Q[qcur] holds the primitive state of U0
@@ -80,6 +110,7 @@ struct amun_ctx {
     double* FB = nullptr;               // averaged fine fluxes per slot
     DevState* dummy = nullptr;          // events of the fine-flux recomputation
   } amr;
+  Staging staging;             // of large downloads (copy_to_host)
   // ghost blocks of the non-periodic domain sides
   struct Bnd {
     bool on = false;
@@ -1014,6 +1045,7 @@ void amun_dev_finalize(amun_ctx* c) {
   if (!c) return;
   if (c->stream) hipStreamSynchronize(c->stream);
   drop_graphs(c);
+  c->staging.drop();
   hipFree(c->tape.ck);
   hipFree(c->tape.ckc);
   hipFree(c->tape.dtc);
@@ -1073,6 +1105,59 @@ static int after_upload(amun_ctx* c, int r0, int nr, bool zero_c = true) {
   return 0;
 }
 
+// n bytes of device memory at src, written by c->stream, to host memory.  The
+// runtime's copy into pageable memory stages it on one thread (10.5 GB/s); from
+// kStagedBytes on, kStagedThreads copy out of pinned pieces while the bus
+// fills others: 1.2 GB 114 -> 31 ms, 465 MB 44 -> 12, 151 MB 14.3 -> 4.3, and
+// 33, 14.5 and 6.3 ms for the first, which pins the pieces.  Two MiB a piece
+// and four threads: one MiB leaves gaps on the bus (39 ms for 1.2 GB), four
+// gain 1.6 ms there and lose as much on a first copy, and so do eight threads.
+// Smaller copies than kStagedBytes gain little over that first 2 ms.
+static int copy_to_host(amun_ctx* c, double* dst, const double* src, size_t n) {
+  Staging& S = c->staging;
+  if (n < kStagedBytes || !S.make()) {
+    HIP_TRY(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    return 0;
+  }
+  int dev = 0;
+  HIP_TRY(hipGetDevice(&dev));
+  const char* const from = reinterpret_cast<const char*>(src);
+  char* const to = reinterpret_cast<char*>(dst);
+  hipError_t err[kStagedThreads] = {};
+  auto work = [&](int t) {
+    const size_t step = kStagedPiece * kStagedThreads;
+    auto piece = [&](int h) { return S.pin + (size_t)(2 * t + h) * kStagedPiece; };
+    auto fetch = [&](int h, size_t o) {
+      const hipError_t e = hipMemcpyAsync(piece(h), from + o, std::min(kStagedPiece, n - o),
+                                          hipMemcpyDeviceToHost, c->stream);
+      return e == hipSuccess ? hipEventRecord(S.done[2 * t + h], c->stream) : e;
+    };
+    hipError_t e = hipSetDevice(dev);
+    size_t o = t * kStagedPiece;
+    if (e == hipSuccess && o < n) e = fetch(0, o);
+    for (int h = 0; e == hipSuccess && o < n; o += step, h ^= 1) {
+      if (o + step < n && (e = fetch(h ^ 1, o + step)) != hipSuccess) break;
+      if ((e = hipEventSynchronize(S.done[2 * t + h])) != hipSuccess) break;
+      std::memcpy(to + o, piece(h), std::min(kStagedPiece, n - o));
+    }
+    err[t] = e;
+  };
+  std::thread th[kStagedThreads];
+  int started = 0;
+  try {
+    for (; started < kStagedThreads - 1; started++) th[started] = std::thread(work, started);
+  } catch (...) {   // no thread to be had: this one does the rest
+  }
+  for (int t = started; t < kStagedThreads; t++) work(t);
+  for (int t = 0; t < started; t++) th[t].join();
+  // nothing is in flight when the pieces are used again, after an error either
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  for (hipError_t e : err)
+    if (e != hipSuccess) return fail(1000 + (int)e, std::string("download: ") + hipGetErrorString(e));
+  return 0;
+}
+
 // Between steps U1 holds nothing (the first stage of every integrator writes
 // it), so the transfers convert in it and allocate nothing.
 static dim3 transfer_grid(long long n) {
@@ -1109,10 +1194,7 @@ static int pool_to_grid(amun_ctx* c, int r, const void* X, size_t es, double* u)
     hipLaunchKernelGGL((k_grid_transfer<float, false>), grid, dim3(256), 0, c->stream,
                        static_cast<const float*>(X), c->U1, run_shape(c, r), c->rc, c->nv);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpyAsync(u, c->U1, (size_t)n / c->rc.ncell * per * sizeof(double),
-                         hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  return 0;
+  return copy_to_host(c, u, c->U1, (size_t)n / c->rc.ncell * per * sizeof(double));
 }
 
 // Calls f(buffer, first block, blocks) over all blocks, with a device buffer
@@ -1177,10 +1259,7 @@ static int download_blocks_virtual(amun_ctx* c, double* u, double* q) {
                              b0, nb);
       });
       HIP_TRY(hipGetLastError());
-      HIP_TRY(hipMemcpyAsync(dst + b0 * per, buf, nb * per * sizeof(double),
-                             hipMemcpyDeviceToHost, c->stream));
-      HIP_TRY(hipStreamSynchronize(c->stream));
-      return 0;
+      return copy_to_host(c, dst + b0 * per, buf, nb * per * sizeof(double));
     });
   }
   return r;
@@ -1222,10 +1301,7 @@ int amun_dev_download_interiors(amun_ctx* c, double* u) {
                        dim3(256), 0, c->stream, (const double*)c->U0, buf, b0, nb, c->rc.nc, 0,
                        c->rc, c->nv);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(u + b0 * per, buf, nb * per * sizeof(double), hipMemcpyDeviceToHost,
-                           c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return 0;
+    return copy_to_host(c, u + b0 * per, buf, nb * per * sizeof(double));
   });
 }
 

@@ -2,7 +2,7 @@
 go wrong: blocks of 4 to 64 cells (odd numbers of 4-cell rows, pencils that do
 not fill a workgroup, workgroups over several blocks), launches on both sides
 of the small-grid rule, adjoint faces over several tiles, fine faces of small
-blocks, and a handful of states."""
+blocks, a handful of states, and downloads on both sides of the staged copy."""
 import ctypes
 
 import numpy as np
@@ -137,3 +137,23 @@ def test_cons2prim_noalloc_sizes(eq, n):
             torch.cuda.current_stream().cuda_stream) == 0
         np.testing.assert_array_equal(dq.cpu().numpy(), ref)
         assert dev.cpu().tolist() == list(ev)
+
+
+@pytest.mark.parametrize("blocks", [(128, 63), (128, 64), (128, 65)])
+def test_download_sizes(blocks):
+    """Four variables of 2048 x 1008, 1024 and 1040 cells: just below, at and
+    beyond (with an incomplete last piece) the 64 MiB of the staged copy.  The
+    state comes back as it went, twice, and after a step as its blocks hold it."""
+    p = _params(2, "hd", "tvd", 16, blocks, equation_of_state="iso", csnd=0.8)
+    p.riemann_solver = "hll"
+    u0 = np.random.default_rng(1).uniform(0.9, 1.1, (4,) + p.shape)
+    with Solver(p) as s:
+        s.upload(u0)
+        for _ in range(2):
+            np.testing.assert_array_equal(s.download(), u0)
+        s.run(1)
+        u, b = s.download(), s.download_blocks()
+    g, n = p.nghosts, p.ncells
+    b = np.asarray(b).reshape(blocks[1], blocks[0], n + 2 * g, n + 2 * g, 4)
+    b = b[:, :, g:g + n, g:g + n].transpose(4, 0, 2, 1, 3).reshape(u.shape)
+    np.testing.assert_array_equal(u, b)
