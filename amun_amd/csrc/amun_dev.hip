@@ -1598,9 +1598,14 @@ static int enqueue_step(amun_ctx* c, double dtnext, int slot, int qcur, hipEvent
       }
       a.swz = c->swz[dir];
       SweepShape w = sweep_shape(c, dir, c->wg[dir]);
-      // a grid that leaves CUs idle: smaller workgroups on more of them (128^2
-      // HD, 74 workgroups of 14 pencils: 42.4 us a step, 171 of 6: 39.7)
-      if (w.grid < kComputeUnits) w = sweep_shape(c, dir, 128);
+      // a grid that leaves CUs idle: smaller workgroups on more of them, until
+      // every CU has one (us a step replayed from graphs with 256, 128, 64
+      // lanes: 128^2 HD 36.7, 34.9, 33.8; with 128 and 64: 64^2 HD 34.6, 32.5,
+      // 64^2 MHD 60.9, 57.1, 16^3 MHD WENO5-Z 76.6, 72.1).  With more
+      // workgroups than CUs the larger ones waste fewer lanes: 512^2 SRMHD y
+      // sweep 75 us with 256, 83 with 128, 106 with 64.
+      for (int wg : {128, 64})
+        if (w.grid < kComputeUnits) w = sweep_shape(c, dir, wg);
       a.np = w.np;
       hipLaunchKernelGGL(d.sweep[dir], dim3(w.grid), dim3(w.lanes), w.lds, c->stream, a, rc);
       parts = (int)w.grid;
