@@ -249,8 +249,8 @@ __global__ __launch_bounds__(256) void k_tlm_face(const double* __restrict__ X, 
 // lF = dxi (MU(i+1) - MU(i)), then AL(i) = (dF/dqL)^T lF, AR(i) = (dF/dqR)^T
 // lF, GF(i) = (dF/dgamma) . lF.
 // A workgroup takes 64 faces: its waves form the face states and lF variable
-// by variable in LDS, then evaluate the Jacobian column by column, each lane
-// one face and one column (Dual<1>: about twice the solver's registers, two
+// by variable in LDS, then evaluate the Jacobian column by column (of
+// blockIdx.y's share of them), each lane one face and one column (Dual<1>: about twice the solver's registers, two
 // waves per SIMD).  Bound by VALU issue.  One lane per face with four columns
 // at a time spilled 2 KB a lane and gave a 128^2 grid a quarter of the
 // chip's SIMDs: 595 us (x) and 637 us (y) a launch at 128^2 MHD HLLD, now
@@ -287,7 +287,7 @@ __global__ __launch_bounds__(256, 2) void k_adj_face(
   // 2NV gamma
   using D1 = Dual<1, TF>;
   const size_t base = (size_t)b * NV * rc.ncell + lidx<8>(rc.nc, rc.nd, i, j, k);
-  for (int n = w; n <= 2 * NV; n += 4) {
+  for (int n = w + 4 * blockIdx.y; n <= 2 * NV; n += 4 * gridDim.y) {
     D1 ql[NV], qr[NV], fl[NV];
 #pragma unroll
     for (int p = 0; p < NV; p++) {
@@ -343,7 +343,7 @@ __global__ void k_tlm_cell(const double* __restrict__ DF0, const double* __restr
 // cons2prim; LT(i) = (dL/dX)^T MU at i, GC(i) = the gamma part of the cell
 // (its cons2prim term plus the flux term of its upper faces)
 template <class P, int ND>
-__global__ __launch_bounds__(256) void k_adj_cell(const double* __restrict__ X, const double* __restrict__ Q,
+__global__ __launch_bounds__(ND == 2 ? 576 : 256) void k_adj_cell(const double* __restrict__ X, const double* __restrict__ Q,
                            const double* __restrict__ AL0, const double* __restrict__ AR0,
                            const double* __restrict__ AL1, const double* __restrict__ AR1,
                            const double* __restrict__ AL2, const double* __restrict__ AR2,
@@ -384,7 +384,7 @@ __global__ __launch_bounds__(256) void k_adj_cell(const double* __restrict__ X, 
       lq += (AL[D][var_index<NV>(rc, pcell[2], v)] - AR[D][var_index<NV>(rc, pface[2], v)]) * dm;
     }
   };
-  for (v = w; active && v < NV; v += 4) {
+  for (v = w; active && v < NV; v += blockDim.x >> 6) {
     lq = 0.0;
     per_dir(std::integral_constant<int, 0>());
     per_dir(std::integral_constant<int, 1>());

@@ -2582,7 +2582,17 @@ int amun_dev_tape_backward(amun_ctx* c, const double* lam, double* lam0, double*
   if ((r = grad_state(c, keep, false))) return r;
   const long long nn = (long long)n;
   const dim3 gc((unsigned)(((long long)ncell + 255) / 256)), bl(256);
-  const dim3 gface((unsigned)((ncell + kAdjFaces - 1) / kAdjFaces));
+  const unsigned gtile = (unsigned)((ncell + kAdjFaces - 1) / kAdjFaces);
+  // Fewer tiles than CUs: the columns of a tile's Jacobian over several
+  // workgroups, each of which forms the face states again (64^2 MHD, six steps:
+  // 3.35 ms in one, 2.69, 2.47 and 2.47 in 2, 3 and 5; 128^2: 3.47 in one, 3.52
+  // in 2; 256^2: 9.3 and 10.7).
+  const dim3 gface(gtile, std::max(1u, std::min((2 * c->nv + 4) / 4u, kComputeUnits / gtile)));
+  // A wave a variable while the tiles are few (64^2, 128^2, 256^2, 512^2 with
+  // four waves and with nine: 3.35, 3.47, 9.26, 30.8 and 2.87, 3.21, 9.02,
+  // 31.6 ms); in 3D its registers let only eight run (32^3: 8.4 and 8.7 ms).
+  const dim3 bcell(64 * (nd == 2 && gtile <= 4 * kComputeUnits ? c->nv : 4));
+  const dim3 ge((unsigned)std::min(2048ll, (nn + 255) / 256));
   if ((r = global_to_pool(c, lam, B.LU0))) return r;     // lambda of U^N
   RunState h;
   HIP_TRY(hipMemcpy(&h, c->rs, sizeof(RunState), hipMemcpyDeviceToHost));
@@ -2593,39 +2603,39 @@ int amun_dev_tape_backward(amun_ctx* c, const double* lam, double* lam0, double*
     for (int s = s1 - 1; s >= s0; s--) {
       const double* X0 = B.seg + (size_t)(s - s0) * ns * n;
       // lambda of the last stage output: psi decay of the step
-      hipLaunchKernelGGL(k_axpby, dim3(2048), bl, 0, c->stream, nn, 1.0, B.LU0, 0.0, B.LY);
+      hipLaunchKernelGGL(k_axpby, ge, bl, 0, c->stream, nn, 1.0, B.LU0, 0.0, B.LY);
       if (c->cfg.eqsys == AMUN_EQSYS_MHD)
-        hipLaunchKernelGGL(k_scale_var, dim3(2048), bl, 0, c->stream, B.LY, c->nv, 7, rc.decay, rc);
-      hipLaunchKernelGGL(k_axpby, dim3(2048), bl, 0, c->stream, nn, 0.0, B.LY, 0.0, B.LU0);
+        hipLaunchKernelGGL(k_scale_var, gc, bl, 0, c->stream, B.LY, c->nv, 7, rc.decay, rc);
+      hipLaunchKernelGGL(k_axpby, ge, bl, 0, c->stream, nn, 0.0, B.LY, 0.0, B.LU0);
       if (ksrc > 0)
-        hipLaunchKernelGGL(k_axpby, dim3(2048), bl, 0, c->stream, nn, 0.0, B.LY, 0.0, B.LS);
+        hipLaunchKernelGGL(k_axpby, ge, bl, 0, c->stream, nn, 0.0, B.LY, 0.0, B.LS);
       for (int k = ns - 1; k >= 0; k--) {
         const double* X = X0 + (size_t)k * n;
         // MU = c dt lambda_Y, LT = (dL/dX)^T MU
-        hipLaunchKernelGGL(k_axpby, dim3(2048), bl, 0, c->stream, nn, co[k].c * T.dt[s], B.LY,
+        hipLaunchKernelGGL(k_axpby, ge, bl, 0, c->stream, nn, co[k].c * T.dt[s], B.LY,
                            0.0, B.MU);
         hipLaunchKernelGGL(d.adj_prim, gc, bl, 0, c->stream, X, B.Q, rc);
         for (int dd = 0; dd < nd; dd++)
           hipLaunchKernelGGL(d.adj_face[dd], gface, bl, 0, c->stream, B.Q, B.MU, B.AL[dd], B.AR[dd],
                              B.GF[dd], c->nbr, rc, h.dxi[dd], T.cmax[s]);
         const int z = nd == 3 ? 2 : 1;
-        hipLaunchKernelGGL(d.adj_cell, gface, bl, 0, c->stream, X, B.Q, B.AL[0], B.AR[0], B.AL[1],
+        hipLaunchKernelGGL(d.adj_cell, dim3(gtile), bcell, 0, c->stream, X, B.Q, B.AL[0], B.AR[0], B.AL[1],
                            B.AR[1], B.AL[z], B.AR[z], B.GF[0], B.GF[1], B.GF[z], B.LT, B.GC,
                            c->nbr, rc);
         hipLaunchKernelGGL(k_sum_acc, dim3(npart), bl, 0, c->stream, B.GC, (long long)ncell, B.GP);
         // lambda of X_src gets a lambda_Y; lambda of X = b lambda_Y + LT
         // (+ what a later stage passed to it as its X_src)
         if (co[k].a != 0.0)
-          hipLaunchKernelGGL(k_axpby, dim3(2048), bl, 0, c->stream, nn, co[k].a, B.LY, 1.0,
+          hipLaunchKernelGGL(k_axpby, ge, bl, 0, c->stream, nn, co[k].a, B.LY, 1.0,
                              co[k].src ? B.LS : B.LU0);
-        hipLaunchKernelGGL(k_axpby, dim3(2048), bl, 0, c->stream, nn, co[k].b, B.LY, 0.0, B.MU);
-        hipLaunchKernelGGL(k_axpby, dim3(2048), bl, 0, c->stream, nn, 1.0, B.LT, 1.0, B.MU);
+        hipLaunchKernelGGL(k_axpby, ge, bl, 0, c->stream, nn, co[k].b, B.LY, 0.0, B.MU);
+        hipLaunchKernelGGL(k_axpby, ge, bl, 0, c->stream, nn, 1.0, B.LT, 1.0, B.MU);
         if (ksrc > 0 && k == ksrc)
-          hipLaunchKernelGGL(k_axpby, dim3(2048), bl, 0, c->stream, nn, 1.0, B.LS, 1.0, B.MU);
+          hipLaunchKernelGGL(k_axpby, ge, bl, 0, c->stream, nn, 1.0, B.LS, 1.0, B.MU);
         if (k == 0)
-          hipLaunchKernelGGL(k_axpby, dim3(2048), bl, 0, c->stream, nn, 1.0, B.MU, 1.0, B.LU0);
+          hipLaunchKernelGGL(k_axpby, ge, bl, 0, c->stream, nn, 1.0, B.MU, 1.0, B.LU0);
         else
-          hipLaunchKernelGGL(k_axpby, dim3(2048), bl, 0, c->stream, nn, 1.0, B.MU, 0.0, B.LY);
+          hipLaunchKernelGGL(k_axpby, ge, bl, 0, c->stream, nn, 1.0, B.MU, 0.0, B.LY);
       }
     }
     HIP_TRY(hipGetLastError());

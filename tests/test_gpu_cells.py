@@ -72,11 +72,13 @@ def test_sweep_sizes_vs_oracle(case, precision):
     assert relerr(ug, uo).max() <= (1e-12 if precision == "fp64" else 4.6e-6)
 
 
-@pytest.mark.parametrize("nd,n,blocks", [(2, 4, (3, 5)), (2, 64, (2, 1)), (3, 4, (3, 2, 2)),
-                                         (3, 12, (2, 1, 2)), (3, 20, (1, 2, 1))])
+@pytest.mark.parametrize("nd,n,blocks", [(2, 4, (3, 5)), (2, 64, (2, 1)), (2, 16, (17, 16)),
+                                         (3, 4, (3, 2, 2)), (3, 12, (2, 1, 2)),
+                                         (3, 20, (1, 2, 1))])
 def test_adjoint_sizes(nd, n, blocks):
     """<lam, T(du0, dg)> = <A(lam), du0> + A_gamma(lam) dg to round-off, at
-    block sizes with fewer and more faces than a tile of the adjoint holds"""
+    block sizes with fewer and more faces than a tile of the adjoint holds, and
+    on both sides of its rules for few tiles"""
     p = _params(nd, "mhd", "tvd", n, blocks)
     print(f"[case] adjoint {nd}D n={n} blocks={blocks}", flush=True)
     u0 = _mhd_state(p, noise=0.01)
