@@ -10,6 +10,8 @@
 
 #include <array>
 #include <map>
+#include <memory>
+#include <mutex>
 #include <thread>
 
 // ===========================================================================
@@ -111,6 +113,10 @@ struct amun_ctx {
     DevState* dummy = nullptr;          // events of the fine-flux recomputation
   } amr;
   Staging staging;             // of large downloads (copy_to_host)
+  // Held while a transfer puts its commands into the stream (and, to the host,
+  // until the copy has ended) and while a step puts in its own: both write U1,
+  // and the transfers of several threads share the staging buffers.
+  std::unique_ptr<std::mutex> busy = std::make_unique<std::mutex>();
   // ghost blocks of the non-periodic domain sides
   struct Bnd {
     bool on = false;
@@ -1159,7 +1165,8 @@ static int copy_to_host(amun_ctx* c, double* dst, const double* src, size_t n) {
 }
 
 // Between steps U1 holds nothing (the first stage of every integrator writes
-// it), so the transfers convert in it and allocate nothing.
+// it), so the transfers convert in it and allocate nothing.  The context's
+// mutex keeps the transfers and steps of several threads apart.
 static dim3 transfer_grid(long long n) {
   return dim3((unsigned)std::max(1ll, std::min(8192ll, (n + 255) / 256)));
 }
@@ -1174,6 +1181,7 @@ static GridShape run_shape(const amun_ctx* c, int r) {
 static int grid_to_pool(amun_ctx* c, int r, const double* u, double* X) {
   const size_t per = (size_t)c->nv * c->rc.ncell;
   const long long n = (long long)(c->run_b0[r + 1] - c->run_b0[r]) * c->rc.ncell;
+  std::lock_guard<std::mutex> hold(*c->busy);
   HIP_TRY(hipMemcpyAsync(c->U1, u, (size_t)n / c->rc.ncell * per * sizeof(double),
                          hipMemcpyHostToDevice, c->stream));
   hipLaunchKernelGGL((k_grid_transfer<double, true>), dim3(transfer_grid(n).x, c->nv), dim3(256),
@@ -1187,6 +1195,7 @@ static int pool_to_grid(amun_ctx* c, int r, const void* X, size_t es, double* u)
   const size_t per = (size_t)c->nv * c->rc.ncell;
   const long long n = (long long)(c->run_b0[r + 1] - c->run_b0[r]) * c->rc.ncell;
   const dim3 grid(transfer_grid(n).x, c->nv);
+  std::lock_guard<std::mutex> hold(*c->busy);
   if (es == sizeof(double))
     hipLaunchKernelGGL((k_grid_transfer<double, false>), grid, dim3(256), 0, c->stream,
                        static_cast<const double*>(X), c->U1, run_shape(c, r), c->rc, c->nv);
@@ -1203,6 +1212,7 @@ static int pool_to_grid(amun_ctx* c, int r, const void* X, size_t es, double* u)
 extern "C++" template <class F>
 static int by_block_chunks(amun_ctx* c, size_t per, F&& f) {
   const int nblk = c->rc.nblk;
+  std::lock_guard<std::mutex> hold(*c->busy);
   if (c->nstate < per) {
     double* buf = nullptr;
     HIP_TRY(hipMalloc((void**)&buf, nblk * per * sizeof(double)));
@@ -1628,6 +1638,7 @@ static int enqueue_step(amun_ctx* c, double dtnext, int slot, int qcur, hipEvent
 // One step: replayed from a captured graph when graphs are on (and no
 // per-kernel events are wanted), launched kernel by kernel otherwise.
 static int launch_step(amun_ctx* c, double dtnext, hipEvent_t* ev = nullptr) {
+  std::lock_guard<std::mutex> hold(*c->busy);
   const int slot = (int)(c->nsteps & 1), qcur = c->qcur;
   if (c->use_graph && !ev) {
     hipGraphExec_t exec = nullptr;
@@ -2247,9 +2258,10 @@ int amun_dev_amr_remesh(amun_ctx* c, int32_t nblk, const int32_t* meta) {
     n->swz[d] = c->swz[d];
   }
   n->use_graph = c->use_graph;
-  // the new context takes the caller's handle and stream
+  // the new context takes the caller's handle, stream and mutex
   std::swap(*c, *n);
   std::swap(c->stream, n->stream);
+  std::swap(c->busy, n->busy);
   amun_dev_finalize(n);
   return after_upload(c, 0, 1, false);
 }
@@ -2418,6 +2430,7 @@ int recompute_segment(amun_ctx* c, int s0, int s1, double* seg) {
     HIP_TRY(hipMemcpyAsync(c->C, T.ckc + (size_t)(s0 / T.interval) * c->nstate,
                            c->nstate * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
   for (int s = s0; s < s1; s++) {
+    std::lock_guard<std::mutex> hold(*c->busy);
     hipLaunchKernelGGL(k_set_fixed, dim3(1), dim3(1), 0, c->stream, c->rs, T.dt[s], T.cmax[s]);
     r = enqueue_step(c, 2.0e30, (int)(c->nsteps & 1), c->qcur, nullptr,
                      seg + (size_t)(s - s0) * ns * c->nstate);
