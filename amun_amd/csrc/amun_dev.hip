@@ -252,7 +252,7 @@ int validate(const amun_cfg& c, int* nv) {
     return fail(500, "glm_source_terms must be 0 (none), 1 (eglm) or 2 (heglm)");
   if (!(c.viscosity >= 0.0) || !(c.resistivity >= 0.0))
     return fail(500, "viscosity and resistivity must be non-negative");
-  if (c.ncells < 4 || c.ncells > 64 || c.ncells % 4)
+  if (c.ncells < kMinCells || c.ncells > kMaxCells || c.ncells % 4)
     return fail(500, "ncells must be a multiple of 4 in [4, 64] (4x4 brick layout)");
   // interior formulas at the faces of cells -1 and ncells (the reference's
   // lower-order end stencils then stay in the outer ghost layers)
@@ -419,31 +419,11 @@ int validate_grid(const amun_cfg& c, const amun_grid& g) {
   return 0;
 }
 
-// launch shape of a sweep along dir: np pencils of nc + 2 lanes each per
-// workgroup, the lanes, the workgroups and the LDS.  Of the even np with at
-// most wg lanes (at least two pencils), the one that leaves the fewest lanes
-// idle: 14 pencils on 252 of 256 lanes at nc = 16.
-struct SweepShape {
-  int np, lanes;
-  unsigned grid;
-  size_t lds;
-};
-
 constexpr unsigned kComputeUnits = 256;
 
-SweepShape sweep_shape(const amun_ctx* c, int dir, int wg) {
-  const RunConst& rc = c->rc;
-  const long long total = (long long)rc.nblk * (rc.nd == 3 ? rc.nc * rc.nc : rc.nc);
-  const auto lanes = [&](int np) { return (np * (rc.nc + 2) + 63) / 64 * 64; };
-  SweepShape s;
-  s.np = 2;
-  for (int np = 2; lanes(np) <= wg; np += 2)
-    if ((long long)np * lanes(s.np) >= (long long)s.np * lanes(np)) s.np = np;
-  s.lanes = lanes(s.np);
-  s.grid = (unsigned)((total + s.np - 1) / s.np);
-  s.lds = sweep_lds_elems(c->nv, (int)c->qsize, relativistic(c->cfg), c->disp.R, rc.nc, s.np, dir) *
-          c->qsize;
-  return s;
+// what the launch shapes of a context's sweeps depend on
+SweepCfg sweep_cfg(const amun_ctx* c) {
+  return {c->nv, (int)c->qsize, relativistic(c->cfg), c->disp.R, c->rc.nd, c->rc.nc, c->rc.nblk};
 }
 
 // the slopes of the multi-dimensional limiting of the stage input Q[qcur]
@@ -740,10 +720,9 @@ static int init_device(amun_ctx* c, const std::vector<int32_t>& nbr,
   }
   // allow the sweeps' LDS (above the 64 KiB default of dynamic LDS)
   for (int dir = 0; dir < nd; dir++) {
-    size_t lds = 0;
-    for (int wg : {64, 128, 256}) lds = std::max(lds, sweep_shape(c, dir, wg).lds);
     e = hipFuncSetAttribute((const void*)c->disp.sweep[dir],
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+                            hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)sweep_lds_limit(sweep_cfg(c), dir));
     if (e != hipSuccess) {
       amun_dev_finalize(c);
       return fail(1000 + (int)e, "hipFuncSetAttribute (LDS)");
@@ -1607,7 +1586,8 @@ static int enqueue_step(amun_ctx* c, double dtnext, int slot, int qcur, hipEvent
                            c->st);
       }
       a.swz = c->swz[dir];
-      SweepShape w = sweep_shape(c, dir, c->wg[dir]);
+      const SweepCfg sc = sweep_cfg(c);
+      SweepShape w = sweep_shape(sc, dir, c->wg[dir]);
       // a grid that leaves CUs idle: smaller workgroups on more of them, until
       // every CU has one (us a step replayed from graphs with 256, 128, 64
       // lanes: 128^2 HD 36.7, 34.9, 33.8; with 128 and 64: 64^2 HD 34.6, 32.5,
@@ -1615,7 +1595,7 @@ static int enqueue_step(amun_ctx* c, double dtnext, int slot, int qcur, hipEvent
       // workgroups than CUs the larger ones waste fewer lanes: 512^2 SRMHD y
       // sweep 75 us with 256, 83 with 128, 106 with 64.
       for (int wg : {128, 64})
-        if (w.grid < kComputeUnits) w = sweep_shape(c, dir, wg);
+        if (w.grid < kComputeUnits) w = sweep_shape(sc, dir, wg);
       a.np = w.np;
       hipLaunchKernelGGL(d.sweep[dir], dim3(w.grid), dim3(w.lanes), w.lds, c->stream, a, rc);
       parts = (int)w.grid;

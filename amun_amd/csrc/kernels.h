@@ -42,6 +42,7 @@
 #pragma once
 
 #include "../../include/amun_dev.h"
+#include "launch.h"
 #include "physics.h"
 #include "srmhd.h"
 
@@ -1099,34 +1100,7 @@ constexpr int sweep_min_waves() {
 
 // Lanes of a sweep workgroup: the interior cells of its np pencils, then the
 // cells before and behind each pencil.
-// LDS, in elements of T: the pencils' primitive state with R + 1 cells beyond
-// each end, then in its place the upper face states, then the fluxes.  The
-// width of a pencil's row is the smallest that spreads the lanes of a wave
-// over all banks: four cells by four pencils (x), four pencils by sixteen
-// cells (y), one cell each (z).
-__host__ __device__ constexpr int row_width(int n, int dir) {
-  return dir == 0 ? (n + 3) / 8 * 8 + 4 : (dir == 1 ? (n + 7) / 16 * 16 + 8 : n | 1);
-}
-__host__ __device__ constexpr int tile_width(int nc, int R, int dir) {
-  return row_width(nc + 2 * (R + 1), dir);
-}
-__host__ __device__ constexpr int face_width(int nc, int dir) { return row_width(nc + 1, dir); }
-// Whether the solver leaves registers for the cell's increment and states
-// (HD, and every FP32 system but the relativistic: at most 10 words a state);
-// where not, the increment of the directions before waits in LDS: read at the
-// update instead, it cost 0.5 ms of a 256^3 FP64 MHD step, and early in
-// registers it spilled.
-__host__ __device__ constexpr bool sweep_loads_early(int nv, int es, bool sr) {
-  return nv * es <= 40 && !sr;
-}
-__host__ __device__ constexpr bool sweep_inc_lds(int nv, int es, bool sr, int R, int dir) {
-  return R > 0 && dir > 0 && !sweep_loads_early(nv, es, sr);
-}
-__host__ __device__ constexpr size_t sweep_lds_elems(int nv, int es, bool sr, int R, int nc,
-                                                     int np, int dir) {
-  const int w = R ? tile_width(nc, R, dir) : face_width(nc, dir);
-  return (size_t)nv * np * (w + (sweep_inc_lds(nv, es, sr, R, dir) ? nc : 0));
-}
+// The layout of their LDS stands in launch.h.
 
 // n / d for 0 <= n < 2^16, d > 0, with rd = 1 / d (exact: the distance of
 // (n + 0.5) / d from an integer is at least 0.5 / d)

@@ -159,3 +159,20 @@ def test_download_sizes(blocks):
     b = np.asarray(b).reshape(blocks[1], blocks[0], n + 2 * g, n + 2 * g, 4)
     b = b[:, :, g:g + n, g:g + n].transpose(4, 0, 2, 1, 3).reshape(u.shape)
     np.testing.assert_array_equal(u, b)
+
+
+def test_contexts_share_a_kernel():
+    """A context of 4-cell blocks (83 KB of LDS a workgroup) steps on after
+    one of 16-cell blocks (39 KB) has taken the same kernels into use."""
+    small, large = (_params(3, "mhd", "weno5z", n, (2, 1, 2)) for n in (4, 16))
+    u0 = _state(small)
+    print("[case] contexts of 4- and 16-cell blocks", flush=True)
+    with Solver(small) as a:
+        a.upload(u0)
+        want = a.run(3), a.download()
+        a.upload(u0)
+        with Solver(large) as b:
+            b.upload(_state(large))
+            b.run(1)
+            np.testing.assert_array_equal(a.run(3), want[0])
+        np.testing.assert_array_equal(a.download(), want[1])
