@@ -1090,6 +1090,27 @@ static int after_upload(amun_ctx* c, int r0, int nr, bool zero_c = true) {
   return 0;
 }
 
+// A transfer on any thread: alone with the context's U1 and staging buffers,
+// and with the device of its stream current, which launches and events ask for
+// (a thread begins on device 0, whatever the context is on).
+struct Transfer {
+  std::lock_guard<std::mutex> hold;
+  int was = -1;   // device to go back to
+  hipError_t err;
+  explicit Transfer(amun_ctx* c) : hold(*c->busy) {
+    int now = 0;
+    hipDevice_t dev = 0;
+    err = hipGetDevice(&now);
+    if (err == hipSuccess) err = hipStreamGetDevice(c->stream, &dev);
+    if (err != hipSuccess || dev == now) return;
+    err = hipSetDevice(dev);
+    if (err == hipSuccess) was = now;
+  }
+  ~Transfer() {
+    if (was >= 0) (void)hipSetDevice(was);
+  }
+};
+
 // n bytes of device memory at src, written by c->stream, to host memory.  The
 // runtime's copy into pageable memory stages it on one thread (10.5 GB/s); from
 // kStagedBytes on, kStagedThreads copy out of pinned pieces while the bus
@@ -1160,7 +1181,8 @@ static GridShape run_shape(const amun_ctx* c, int r) {
 static int grid_to_pool(amun_ctx* c, int r, const double* u, double* X) {
   const size_t per = (size_t)c->nv * c->rc.ncell;
   const long long n = (long long)(c->run_b0[r + 1] - c->run_b0[r]) * c->rc.ncell;
-  std::lock_guard<std::mutex> hold(*c->busy);
+  Transfer t(c);
+  HIP_TRY(t.err);
   HIP_TRY(hipMemcpyAsync(c->U1, u, (size_t)n / c->rc.ncell * per * sizeof(double),
                          hipMemcpyHostToDevice, c->stream));
   hipLaunchKernelGGL((k_grid_transfer<double, true>), dim3(transfer_grid(n).x, c->nv), dim3(256),
@@ -1174,7 +1196,8 @@ static int pool_to_grid(amun_ctx* c, int r, const void* X, size_t es, double* u)
   const size_t per = (size_t)c->nv * c->rc.ncell;
   const long long n = (long long)(c->run_b0[r + 1] - c->run_b0[r]) * c->rc.ncell;
   const dim3 grid(transfer_grid(n).x, c->nv);
-  std::lock_guard<std::mutex> hold(*c->busy);
+  Transfer t(c);
+  HIP_TRY(t.err);
   if (es == sizeof(double))
     hipLaunchKernelGGL((k_grid_transfer<double, false>), grid, dim3(256), 0, c->stream,
                        static_cast<const double*>(X), c->U1, run_shape(c, r), c->rc, c->nv);
@@ -1191,7 +1214,8 @@ static int pool_to_grid(amun_ctx* c, int r, const void* X, size_t es, double* u)
 extern "C++" template <class F>
 static int by_block_chunks(amun_ctx* c, size_t per, F&& f) {
   const int nblk = c->rc.nblk;
-  std::lock_guard<std::mutex> hold(*c->busy);
+  Transfer t(c);
+  HIP_TRY(t.err);
   if (c->nstate < per) {
     double* buf = nullptr;
     HIP_TRY(hipMalloc((void**)&buf, nblk * per * sizeof(double)));

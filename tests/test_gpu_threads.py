@@ -5,6 +5,7 @@ import threading
 
 import numpy as np
 import pytest
+import torch   # before the library: one HIP runtime in the process
 
 from amun_amd.problems import kelvin_helmholtz_2d
 from amun_amd.solver import Batch, Solver
@@ -82,3 +83,17 @@ def test_download_while_stepping(case, graph):
         np.testing.assert_array_equal(s.download(), states[-1])
     for u in seen:
         assert any(np.array_equal(u, v) for v in states)
+
+
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="needs two devices")
+def test_large_download_from_a_thread_on_another_device():
+    p = _params(3, "mhd", "weno5z", 16, (7, 6, 6))
+    u0 = _state(p)
+    print("[case] download on another device's thread", flush=True)
+    with torch.cuda.device(1), Solver(p) as s:
+        s.upload(u0)
+        got = []
+        _together([lambda: got.extend(s.download() for _ in range(2))])
+        for u in got:
+            np.testing.assert_array_equal(u, u0)
+        assert torch.cuda.current_device() == 1
