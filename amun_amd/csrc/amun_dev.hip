@@ -79,9 +79,10 @@ struct amun_ctx {
   std::vector<int32_t> run_b0;      // first block of every run (+ total)
   std::vector<int32_t> coords;      // block coordinates inside its run
   Dispatch disp;
-  // launch shapes of the sweeps (workgroup size, XCD-aware order), per
-  // direction; set by amun_dev_autotune
-  int wg[3] = {256, 256, 256};
+  // launch shapes of the sweeps (workgroup size, 0 = by the grid, see
+  // launch_shape; XCD-aware order), per direction; set by amun_dev_autotune
+  // and amun_dev_set_launch
+  int wg[3] = {0, 0, 0};
   int swz[3] = {1, 1, 1};
   // captured steps: one graph per (cmax slot, primitive buffer, dtnext)
   bool use_graph = false;
@@ -418,8 +419,6 @@ int validate_grid(const amun_cfg& c, const amun_grid& g) {
     return fail(500, "domain bounds must be increasing");
   return 0;
 }
-
-constexpr unsigned kComputeUnits = 256;
 
 // what the launch shapes of a context's sweeps depend on
 SweepCfg sweep_cfg(const amun_ctx* c) {
@@ -1610,16 +1609,7 @@ static int enqueue_step(amun_ctx* c, double dtnext, int slot, int qcur, hipEvent
                            c->st);
       }
       a.swz = c->swz[dir];
-      const SweepCfg sc = sweep_cfg(c);
-      SweepShape w = sweep_shape(sc, dir, c->wg[dir]);
-      // a grid that leaves CUs idle: smaller workgroups on more of them, until
-      // every CU has one (us a step replayed from graphs with 256, 128, 64
-      // lanes: 128^2 HD 36.7, 34.9, 33.8; with 128 and 64: 64^2 HD 34.6, 32.5,
-      // 64^2 MHD 60.9, 57.1, 16^3 MHD WENO5-Z 76.6, 72.1).  With more
-      // workgroups than CUs the larger ones waste fewer lanes: 512^2 SRMHD y
-      // sweep 75 us with 256, 83 with 128, 106 with 64.
-      for (int wg : {128, 64})
-        if (w.grid < kComputeUnits) w = sweep_shape(sc, dir, wg);
+      const SweepShape w = launch_shape(sweep_cfg(c), dir, c->wg[dir]);
       a.np = w.np;
       hipLaunchKernelGGL(d.sweep[dir], dim3(w.grid), dim3(w.lanes), w.lds, c->stream, a, rc);
       parts = (int)w.grid;
@@ -1854,15 +1844,15 @@ int amun_dev_autotune(amun_ctx* c, int32_t nsteps, int32_t* choice) {
   c->use_graph = false;
   const int wgs[3] = {64, 128, 256};
   double best[3] = {1e300, 1e300, 1e300};
-  int bwg[3] = {256, 256, 256}, bsw[3] = {1, 1, 1};
+  int bwg[3] = {0, 0, 0}, bsw[3] = {1, 1, 1};
   const int nk = kernels_per_step(c);
   std::vector<double> kms(nk);
   int r = 0;
-  // the x and y sweeps keep workgroups of kSweepLanes lanes
+  // the size of the x and y sweeps' workgroups goes by the grid
   for (int w = 0; w < 3 && !r; w++)
     for (int z = 0; z < 2 && !r; z++) {
       for (int dir = 0; dir < nd; dir++) {
-        c->wg[dir] = dir < 2 ? kSweepLanes : wgs[w];
+        c->wg[dir] = dir < 2 ? 0 : wgs[w];
         c->swz[dir] = z;
       }
       double ms = 0.0;
@@ -1884,7 +1874,7 @@ int amun_dev_autotune(amun_ctx* c, int32_t nsteps, int32_t* choice) {
   if (r) return r;
   if (choice)
     for (int dir = 0; dir < nd; dir++) {
-      choice[2 * dir] = bwg[dir];
+      choice[2 * dir] = dir < 2 ? kSweepLanes : bwg[dir];
       choice[2 * dir + 1] = bsw[dir];
     }
   return 0;
@@ -1900,7 +1890,7 @@ int amun_dev_set_launch(amun_ctx* c, const int32_t* choice) {
   }
   HIP_TRY(hipStreamSynchronize(c->stream));
   for (int dir = 0; dir < c->rc.nd; dir++) {
-    c->wg[dir] = choice[2 * dir];
+    c->wg[dir] = dir < 2 ? 0 : choice[2 * dir];
     c->swz[dir] = choice[2 * dir + 1] != 0;
   }
   drop_graphs(c);

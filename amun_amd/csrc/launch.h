@@ -64,6 +64,22 @@ constexpr SweepShape sweep_shape(const SweepCfg& c, int dir, int wg) {
   return s;
 }
 
+// The shape that a sweep is launched with.  A workgroup size that was chosen
+// (amun_dev_set_launch, amun_dev_autotune) holds.  wg = 0, the default: 256,
+// and on a grid that leaves CUs idle with it 128, then 64, until every CU has
+// a workgroup (us a step replayed from graphs with 256, 128, 64 lanes: 128^2
+// HD 36.7, 34.9, 33.8; with 128 and 64: 64^2 HD 34.6, 32.5, 64^2 MHD 60.9,
+// 57.1, 16^3 MHD WENO5-Z 76.6, 72.1).  With more workgroups than CUs the
+// larger ones waste fewer lanes: 512^2 SRMHD y sweep 75 us with 256, 83 with
+// 128, 106 with 64.
+constexpr unsigned kComputeUnits = 256;
+constexpr SweepShape launch_shape(const SweepCfg& c, int dir, int wg) {
+  if (wg) return sweep_shape(c, dir, wg);
+  SweepShape s = sweep_shape(c, dir, 256);
+  for (int w = 128; w >= 64 && s.grid < kComputeUnits; w /= 2) s = sweep_shape(c, dir, w);
+  return s;
+}
+
 // The largest LDS of any launch of a sweep kernel, over the block sizes that a
 // context may have and the three workgroup sizes.  The limit of dynamic LDS
 // belongs to the kernel, which all contexts of a process share: set to one

@@ -272,11 +272,14 @@ int  amun_dev_statistics_run(amun_ctx* ctx, int32_t r, double out[21]);
 int  amun_dev_set_graph(amun_ctx* ctx, int32_t enable);
 
 /* Launch-shape autotuner: runs nsteps timed steps of the live state for every
- * candidate shape (workgroup of 64, 128 or 256 lanes; plain or XCD-grouped
- * workgroup order), keeps the fastest per sweep direction and restores the
- * state, so the run continues as if the call had not happened.  choice (may
- * be NULL) receives ndims pairs (workgroup size, XCD grouping).
- * amun_dev_set_launch sets such pairs directly. */
+ * candidate shape (z sweep: workgroup of 64, 128 or 256 lanes; every sweep:
+ * plain or XCD-grouped workgroup order), keeps the fastest per sweep direction
+ * and restores the state, so the run continues as if the call had not
+ * happened.  choice (may be NULL) receives ndims pairs (workgroup size, XCD
+ * grouping).  amun_dev_set_launch sets such pairs directly: the size of the z
+ * sweep's workgroups (at least two pencils) then holds on every grid.  The x
+ * and y sweeps take 256 only, the most lanes they run: a grid that leaves
+ * CUs idle runs 128 or 64 there, and in z until a size is set. */
 int  amun_dev_autotune(amun_ctx* ctx, int32_t nsteps, int32_t* choice);
 
 /* Per-stage timing (no reference counterpart; the reference's evolve_* calls

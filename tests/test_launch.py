@@ -58,3 +58,44 @@ def test_lds_limit_does_not_depend_on_the_block_size(shapes):
     for nd, nv, es, sr, R, d, nc, wg, np_, lanes, grid, lds, limit in shapes:
         assert lds <= limit <= 160 * 1024
         assert limits.setdefault((nd, nv, es, sr, R, d), limit) == limit
+
+
+RULE = r"""
+#include <cstdio>
+#include <initializer_list>
+#include "launch.h"
+using namespace amun_dev;
+int main() {
+  for (int nd = 2; nd <= 3; nd++)
+    for (int nc : {4, 8, 16, 64})
+      for (int nblk : {1, 7, 64, 146, 147, 300, 4096})
+        for (int dir = 0; dir < nd; dir++) {
+          const SweepCfg c{9, 8, false, 2, nd, nc, nblk};
+          for (int wg : {0, 64, 128, 256}) {
+            const SweepShape s = launch_shape(c, dir, wg);
+            std::printf("%d %d %u", wg, s.np, s.grid);
+            for (int k : {64, 128, 256}) {
+              const SweepShape t = sweep_shape(c, dir, k);
+              std::printf(" %d %u", t.np, t.grid);
+            }
+            std::printf("\n");
+          }
+        }
+}
+"""
+
+
+def test_a_chosen_workgroup_size_holds(tmp_path):
+    """Chosen sizes run as chosen on every grid; the default is the largest
+    size that gives every CU a workgroup, the smallest where none does."""
+    small = 0
+    for line in _run(tmp_path, RULE).splitlines():
+        wg, np_, grid, *by = [int(x) for x in line.split()]
+        size = {64: by[:2], 128: by[2:4], 256: by[4:]}
+        small += size[256][1] < 256
+        if wg:
+            assert [np_, grid] == size[wg]
+        else:
+            want = next((k for k in (256, 128, 64) if size[k][1] >= 256), 64)
+            assert [np_, grid] == size[want]
+    assert small
