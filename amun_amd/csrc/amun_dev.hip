@@ -2252,10 +2252,11 @@ int amun_dev_amr_remesh(amun_ctx* c, int32_t nblk, const int32_t* meta) {
     n->swz[d] = c->swz[d];
   }
   n->use_graph = c->use_graph;
-  // the new context takes the caller's handle, stream and mutex
+  // the new context takes the caller's handle, stream, mutex and pinned pieces
   std::swap(*c, *n);
   std::swap(c->stream, n->stream);
   std::swap(c->busy, n->busy);
+  std::swap(c->staging, n->staging);
   amun_dev_finalize(n);
   return after_upload(c, 0, 1, false);
 }

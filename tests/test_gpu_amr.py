@@ -5,6 +5,7 @@ after the fill (restriction, prolongation), one step of several
 configurations (<= 1e-12 relative), the reference's multi-step runs from
 the golden fixtures, conservation through the flux correction, mixed
 precision, and HIP-graph replay."""
+import ctypes
 import os
 
 import numpy as np
@@ -547,3 +548,28 @@ def test_c3_amr_adapts_on_device(precision):
         e = relerr(ur.reshape(-1, p.nv), uc.reshape(-1, p.nv))
         print(f"  refine + derefine of {len(lev1)} leaves: max rel {e.max():.2e}")
         assert e.max() <= 1e-14
+
+
+def test_staging_buffers_outlive_a_mesh_update():
+    """The pinned pieces of large downloads (16 MiB, from the first of them to
+    the end of the context) stay through amun_dev_amr_remesh: the mappings
+    that the first large download made are there after an update."""
+    def mappings():
+        with open("/proc/self/maps") as f:
+            spans = [line.split()[0].split("-") for line in f]
+        return {(int(a, 16), int(b, 16)) for a, b in spans}
+    p, meta = mesh.c3_amr_params("fp64", nb=3, r=0.3)
+    u0 = mesh.block_state(p, meta, mesh.blast_prim(p, r0=0.2, seed=1))
+    assert u0.nbytes >= 64 << 20
+    print(f"[case] staging over a mesh update, blocks={len(meta)}", flush=True)
+    with AmrSolver(p, meta) as s:
+        s.upload(u0)
+        before = mappings()
+        out = np.empty_like(u0)
+        s._check(s.lib.amun_dev_download_interiors(s.h, out.ctypes.data_as(
+            ctypes.POINTER(ctypes.c_double))))
+        pinned = [m for m in mappings() - before if m[1] - m[0] == 16 << 20]
+        s.remesh(meta)
+        now = mappings()
+        print("[case] mappings (MiB)", [(b - a) / 2**20 for a, b in pinned], flush=True)
+        assert pinned and all(any(a <= m[0] and m[1] <= b for a, b in now) for m in pinned)
