@@ -1190,13 +1190,31 @@ static int grid_to_pool(amun_ctx* c, int r, const double* u, double* X) {
   return 0;
 }
 
+// A run up to here comes over as blocks and is converted on the host: the
+// conversion on the device is one launch more for the copy to wait for (us a
+// download, host and device: 18 KB 12, 24; 72 KB 18, 26; 162 KB 27.4, 30; 288
+// KB 44, 36).  hipMemcpy and not the asynchronous copy, which takes 9 us more
+// below 16 KB.
+constexpr size_t kHostBytes = (size_t)192 << 10;
+
 // run r of the pool X (element size es) into the global array u on the host
 static int pool_to_grid(amun_ctx* c, int r, const void* X, size_t es, double* u) {
   const size_t per = (size_t)c->nv * c->rc.ncell;
   const long long n = (long long)(c->run_b0[r + 1] - c->run_b0[r]) * c->rc.ncell;
+  const size_t bytes = (size_t)n / c->rc.ncell * per * sizeof(double);
   const dim3 grid(transfer_grid(n).x, c->nv);
   Transfer t(c);
   HIP_TRY(t.err);
+  if (bytes <= kHostBytes) {
+    std::vector<double> h(bytes / sizeof(double));
+    const GridShape s = run_shape(c, r);
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    HIP_TRY(hipMemcpy(h.data(), static_cast<const char*>(X) + s.b0 * per * es,
+                      bytes / sizeof(double) * es, hipMemcpyDeviceToHost));
+    if (es == sizeof(double)) blocks_to_grid(s, c->rc, c->nv, h.data(), u);
+    else blocks_to_grid(s, c->rc, c->nv, reinterpret_cast<const float*>(h.data()), u);
+    return 0;
+  }
   if (es == sizeof(double))
     hipLaunchKernelGGL((k_grid_transfer<double, false>), grid, dim3(256), 0, c->stream,
                        static_cast<const double*>(X), c->U1, run_shape(c, r), c->rc, c->nv);
@@ -1204,7 +1222,7 @@ static int pool_to_grid(amun_ctx* c, int r, const void* X, size_t es, double* u)
     hipLaunchKernelGGL((k_grid_transfer<float, false>), grid, dim3(256), 0, c->stream,
                        static_cast<const float*>(X), c->U1, run_shape(c, r), c->rc, c->nv);
   HIP_TRY(hipGetLastError());
-  return copy_to_host(c, u, c->U1, (size_t)n / c->rc.ncell * per * sizeof(double));
+  return copy_to_host(c, u, c->U1, bytes);
 }
 
 // Calls f(buffer, first block, blocks) over all blocks, with a device buffer

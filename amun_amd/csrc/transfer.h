@@ -40,6 +40,24 @@ static __global__ __launch_bounds__(256) void k_grid_transfer(
   }
 }
 
+// a run's blocks at h, a host copy of its part of the pool, into its global
+// array u (small runs, see kHostBytes)
+template <typename T>
+static void blocks_to_grid(const GridShape& s, const RunConst& rc, int nv, const T* h, double* u) {
+  const int nc = rc.nc, kn = rc.nd == 3 ? nc : 1;
+  const size_t nx = (size_t)s.ir * nc, ny = (size_t)s.jr * nc, nz = (size_t)s.kr * kn;
+  for (int b = 0; b < s.ir * s.jr * s.kr; b++) {
+    const size_t x0 = (size_t)(b % s.ir) * nc, y0 = (size_t)(b / s.ir % s.jr) * nc;
+    const size_t z0 = (size_t)(b / (s.ir * s.jr)) * kn;
+    for (int v = 0; v < nv; v++, h += rc.ncell)
+      for (int k = 0; k < kn; k++)
+        for (int j = 0; j < nc; j++) {
+          double* row = u + ((v * nz + z0 + k) * ny + y0 + j) * nx + x0;
+          for (int i = 0; i < nc; i++) row[i] = double(h[lidx<sizeof(T)>(nc, rc.nd, i, j, k)]);
+        }
+  }
+}
+
 // conserved state of blocks b0 .. b0 + nb - 1 to and from arrays of m^d cells
 // a block, variables fastest, of which the first ng along each axis lie
 // before the interior (ng = 0 and m = nc: interiors); to the pool, the ghost

@@ -176,3 +176,27 @@ def test_contexts_share_a_kernel():
             b.run(1)
             np.testing.assert_array_equal(a.run(3), want[0])
         np.testing.assert_array_equal(a.download(), want[1])
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("nd,eq,n,blocks", [(2, "hd", 4, (1, 1)), (2, "mhd", 16, (3, 1)),
+                                            (2, "hd", 4, (12, 25)), (2, "hd", 4, (7, 43)),
+                                            (3, "mhd", 4, (3, 2, 5)), (3, "hd", 16, (1, 1, 1)),
+                                            (3, "mhd", 12, (2, 1, 1)), (3, "mhd", 4, (43, 1, 1))])
+def test_small_download_sizes(nd, eq, n, blocks, precision):
+    """States below, next to (187.5 and 188.1 of 192 KiB; 193.5) and above the
+    size that is converted on the host, with their primitives: the values that
+    the block arrays hold."""
+    p = _params(nd, eq, "tvd", n, blocks, precision)
+    print(f"[case] small download {nd}D {eq} n={n} blocks={blocks} {precision}", flush=True)
+    with Solver(p) as s:
+        s.upload(_state(p))
+        s.run(1)
+        got = s.download(with_q=True)
+        blk = s.download_blocks(with_q=True)
+    bx, by, bz = (blocks + (1,))[:3]
+    g, kn = p.nghosts, n if nd == 3 else 1
+    for a, b in zip(got, blk):
+        b = b.reshape((bz, by, bx) + b.shape[1:])[:, :, :, g if nd == 3 else 0:][:, :, :, :kn]
+        b = b[:, :, :, :, g:g + n, g:g + n].transpose(6, 0, 3, 1, 4, 2, 5)
+        np.testing.assert_array_equal(a, b.reshape(a.shape))
