@@ -58,6 +58,20 @@ static void blocks_to_grid(const GridShape& s, const RunConst& rc, int nv, const
   }
 }
 
+// the interiors h of nblk host blocks u with ng ghost layers, variables
+// fastest: a row of cells is contiguous in both
+static void interiors_of(const RunConst& rc, int nv, int ng, int nblk, const double* u,
+                         double* h) {
+  const int nc = rc.nc, m = nc + 2 * ng;
+  const int kn = rc.nd == 3 ? nc : 1, km = rc.nd == 3 ? m : 1, kg = rc.nd == 3 ? ng : 0;
+  const size_t row = (size_t)nc * nv;
+  for (int b = 0; b < nblk; b++)
+    for (int k = 0; k < kn; k++)
+      for (int j = 0; j < nc; j++, h += row)
+        std::memcpy(h, u + ((((size_t)b * km + (k + kg)) * m + (j + ng)) * m + ng) * nv,
+                    row * sizeof(double));
+}
+
 // conserved state of blocks b0 .. b0 + nb - 1 to and from arrays of m^d cells
 // a block, variables fastest, of which the first ng along each axis lie
 // before the interior (ng = 0 and m = nc: interiors); to the pool, the ghost

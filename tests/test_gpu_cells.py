@@ -200,3 +200,32 @@ def test_small_download_sizes(nd, eq, n, blocks, precision):
         b = b.reshape((bz, by, bx) + b.shape[1:])[:, :, :, g if nd == 3 else 0:][:, :, :, :kn]
         b = b[:, :, :, :, g:g + n, g:g + n].transpose(6, 0, 3, 1, 4, 2, 5)
         np.testing.assert_array_equal(a, b.reshape(a.shape))
+
+
+@pytest.mark.parametrize("nd,eq,n,blocks", [(2, "hd", 4, (1, 1)), (2, "mhd", 32, (1, 1)),
+                                            (2, "mhd", 16, (12, 11)), (2, "mhd", 32, (8, 8)),
+                                            (3, "hd", 8, (5, 5, 5)), (3, "hd", 4, (24, 24, 12)),
+                                            (2, "mhd", 16, (32, 32)), (3, "mhd", 8, (10, 9, 10))])
+def test_block_upload_sizes(nd, eq, n, blocks):
+    """Block arrays with ghost layers on both sides of the rule that gathers
+    their interiors on the host (0.6 KB to 33 MB; ghost layers of 0.3 to 7
+    times the interiors): the state of the interiors, whatever the ghost cells
+    hold."""
+    p = _params(nd, eq, "tvd", n, blocks)
+    print(f"[case] block upload {nd}D {eq} n={n} blocks={blocks}", flush=True)
+    u0 = _state(p)
+    g = p.nghosts
+    bx, by, bz = (blocks + (1,))[:3]
+    gk, kn = (g, n) if nd == 3 else (0, 1)
+    inner = u0.reshape(p.nv, bz, kn, by, n, bx, n).transpose(1, 3, 5, 2, 4, 6, 0)
+    with Solver(p) as s:
+        ub = np.full(s._block_shape(), np.nan)
+        ub[:, gk:gk + kn, g:g + n, g:g + n] = inner.reshape(-1, kn, n, n, p.nv)
+        for _ in range(2):
+            s.upload_blocks(ub)
+            np.testing.assert_array_equal(s.download(), u0)
+            s.run(1)
+        got = s.download()
+        s.upload(u0)
+        s.run(1)
+        np.testing.assert_array_equal(got, s.download())
