@@ -1283,6 +1283,8 @@ static int ghosted_to_pool(amun_ctx* c, const double* u, std::unique_ptr<double[
   return blocks_to_pool(c, h.get(), c->rc.nc, 0);
 }
 
+constexpr size_t kWholeBytes = (size_t)16 << 20, kPairBytes = (size_t)256 << 10;
+
 // Block arrays with ghost layers where ghosts come from virtual blocks
 // (multi-level meshes, non-periodic sides): u from U0 and, in the ghost
 // layers, prim2cons of q's; q from the primitive pool filled from the
@@ -1292,24 +1294,53 @@ static int download_blocks_virtual(amun_ctx* c, double* u, double* q) {
   const int ng = c->cfg.nghosts, im = rc.nc + 2 * ng;
   const size_t per = (size_t)c->nv * im * im * (rc.nd == 3 ? im : 1);
   int r = c->amr.on ? amr_fill(c, c->qcur, (int)(c->nsteps & 1)) : bnd_fill(c, c->qcur);
+  if (r) return r;
+  const auto pack = [&](const double* U, double* buf, int b0, int nb) {
+    const dim3 grid = transfer_grid((long long)(nb * per / c->nv));
+    by_system(c->cfg, [&](auto tag) {
+      using P = decltype(tag);
+      if (c->qsize == sizeof(double))
+        hipLaunchKernelGGL((k_blocks_ghosts<P, double>), grid, dim3(256), 0, c->stream,
+                           static_cast<const double*>(c->Q[c->qcur]), U, buf, c->nbr, rc, ng, b0,
+                           nb);
+      else
+        hipLaunchKernelGGL((k_blocks_ghosts<P, float>), grid, dim3(256), 0, c->stream,
+                           static_cast<const float*>(c->Q[c->qcur]), U, buf, c->nbr, rc, ng, b0,
+                           nb);
+    });
+    return hipGetLastError();
+  };
+  // Arrays that U1 does not hold go through it in pieces, each of which waits
+  // for the one before.  Small ones take an allocation instead, and the
+  // smallest one copy for both (us a download of u and q: 28 blocks of 8^2
+  // MHD of three levels 200 in pieces, 111 with an allocation; four of 16^2
+  // HD with open sides 101, 58, and 41 with one copy).
+  const size_t n = rc.nblk * per, bytes = n * sizeof(double);
+  if (bytes <= kWholeBytes) {
+    Transfer t(c);
+    HIP_TRY(t.err);
+    double* buf = nullptr;
+    HIP_TRY(hipMalloc((void**)&buf, (q ? 2 : 1) * bytes));
+    hipError_t e = pack(c->U0, buf, 0, rc.nblk);
+    if (e == hipSuccess && q) e = pack(nullptr, buf + n, 0, rc.nblk);
+    if (e == hipSuccess && q && bytes <= kPairBytes) {
+      std::unique_ptr<double[]> h(new double[2 * n]);
+      e = hipMemcpyAsync(h.get(), buf, 2 * bytes, hipMemcpyDeviceToHost, c->stream);
+      if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+      std::memcpy(u, h.get(), bytes);
+      std::memcpy(q, h.get() + n, bytes);
+    } else if (e == hipSuccess) {
+      r = copy_to_host(c, u, buf, bytes);
+      if (!r && q) r = copy_to_host(c, q, buf + n, bytes);
+    }
+    (void)hipFree(buf);
+    return e == hipSuccess ? r : fail(1000 + (int)e, "download_blocks");
+  }
   for (int pass = 0; pass < 2 && !r; pass++) {
     double* dst = pass == 0 ? u : q;
     if (!dst) continue;
-    const double* U = pass == 0 ? c->U0 : nullptr;
     r = by_block_chunks(c, per, [&](double* buf, int b0, int nb) -> int {
-      const dim3 grid = transfer_grid((long long)(nb * per / c->nv));
-      by_system(c->cfg, [&](auto tag) {
-        using P = decltype(tag);
-        if (c->qsize == sizeof(double))
-          hipLaunchKernelGGL((k_blocks_ghosts<P, double>), grid, dim3(256), 0, c->stream,
-                             static_cast<const double*>(c->Q[c->qcur]), U, buf, c->nbr, rc, ng,
-                             b0, nb);
-        else
-          hipLaunchKernelGGL((k_blocks_ghosts<P, float>), grid, dim3(256), 0, c->stream,
-                             static_cast<const float*>(c->Q[c->qcur]), U, buf, c->nbr, rc, ng,
-                             b0, nb);
-      });
-      HIP_TRY(hipGetLastError());
+      HIP_TRY(pack(pass == 0 ? c->U0 : nullptr, buf, b0, nb));
       return copy_to_host(c, dst + b0 * per, buf, nb * per * sizeof(double));
     });
   }

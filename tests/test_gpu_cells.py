@@ -229,3 +229,29 @@ def test_block_upload_sizes(nd, eq, n, blocks):
         s.upload(u0)
         s.run(1)
         np.testing.assert_array_equal(got, s.download())
+
+
+@pytest.mark.parametrize("blocks", [(3, 3), (12, 11), (40, 38)])
+def test_ghosted_download_sizes(blocks):
+    """Block arrays of an open domain in one copy (u and q of 141 KB each), in
+    one piece (2.1 MB) and in several (24 MB): u alone and with q, interiors
+    as the global arrays hold them, ghost layers as the neighbours do."""
+    p = _params(2, "hd", "tvd", 16, blocks)
+    p.xlbndry = p.xubndry = p.ylbndry = p.yubndry = "open"
+    print(f"[case] ghosted download blocks={blocks}", flush=True)
+    with Solver(p) as s:
+        s.upload(_state(p))
+        s.run(1)
+        glob = s.download(with_q=True)
+        u = s.download_blocks()
+        blk = s.download_blocks(with_q=True)
+    np.testing.assert_array_equal(u, blk[0])
+    g, n, (bx, by) = p.nghosts, p.ncells, blocks
+    u, q = (b.reshape(by, bx, n + 2 * g, n + 2 * g, p.nv) for b in blk)
+    for b, a in zip((u, q), glob):
+        b = b[:, :, g:g + n, g:g + n].transpose(4, 0, 2, 1, 3)
+        np.testing.assert_array_equal(b.reshape(a.shape), a)
+    np.testing.assert_array_equal(q[:, 1:, g:-g, :g], q[:, :-1, g:-g, n:n + g])
+    np.testing.assert_array_equal(q[:-1, :, n + g:, g:-g], q[1:, :, g:2 * g, g:-g])
+    np.testing.assert_array_equal(q[:, 0, g:-g, 0], q[:, 0, g:-g, g])      # open side
+    np.testing.assert_allclose(u[:, 1:, g:-g, :g], u[:, :-1, g:-g, n:n + g], rtol=1e-14, atol=1e-15)
