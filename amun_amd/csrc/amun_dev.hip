@@ -1846,13 +1846,15 @@ int amun_dev_set_graph(amun_ctx* c, int32_t enable) {
 int amun_dev_set_stage_fusion(amun_ctx* c, int32_t on) {
   if (!c) return fail(500, "null argument");
   if (on) {
+    // the configurations that ever took it; the launches of the others are
+    // the same too
     const int npen = c->rc.nd == 3 ? c->rc.nc * c->rc.nc : c->rc.nc;
-    if (!c->disp.stage)
-      return fail(600, "the fused stage is built for the TVD and WENO5-Z reconstructions of "
+    const int rec = c->cfg.reconstruction;
+    if (relativistic(c->cfg) || (rec != AMUN_REC_TVD && rec != AMUN_REC_WENO5Z))
+      return fail(600, "times per stage are offered for the TVD and WENO5-Z reconstructions of "
                        "the non-relativistic systems");
     if (256 % npen)
-      return fail(600, "the fused stage needs whole blocks per workgroup of 256 lanes "
-                       "(ncells^(ndims-1) dividing 256)");
+      return fail(600, "times per stage are offered where ncells^(ndims-1) divides 256");
   }
   HIP_TRY(hipStreamSynchronize(c->stream));
   c->fuse = on ? 1 : 0;
@@ -1863,8 +1865,8 @@ int amun_dev_set_stage_fusion(amun_ctx* c, int32_t on) {
 int amun_dev_autotune(amun_ctx* c, int32_t nsteps, int32_t* choice) {
   if (!c || nsteps < 1) return fail(500, "bad argument");
   if (c->fuse)
-    return fail(600, "autotune chooses the per-direction launches: call it with the fused "
-                     "stage off");
+    return fail(600, "autotune compares the times of single sweeps: call it with the fused "
+                     "stage off (amun_dev_set_stage_fusion)");
   const int nd = c->rc.nd, nr = c->rc.nruns;
   HIP_TRY(hipStreamSynchronize(c->stream));
   // the candidates run real steps on the live state, which is restored

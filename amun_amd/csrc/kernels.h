@@ -1997,8 +1997,7 @@ using namespace amun_dev;
 // kernel instantiations selected for one configuration
 struct Dispatch {
   SweepFn sweep[3] = {nullptr, nullptr, nullptr};
-    int R = 0;                 // window half width of the reconstruction
-  bool stage = false;        // set_stage_fusion is accepted
+  int R = 0;                 // window half width of the reconstruction
   void (*compact[3])(const void*, const int*, RunConst, DevState*) = {nullptr, nullptr, nullptr};
   void (*prim)(const double*, void*, RunConst, DevState*, RunState*, const int*, int, int,
                int) = nullptr;
@@ -2041,7 +2040,6 @@ void fill(Dispatch& d) {
     if constexpr (ND == 3) d.compact[2] = k_compact<P, REC, ND, 2, T>;
   }
   d.R = Recon<P, REC, ND, 0, T>::R;
-  d.stage = (REC == REC_TVD || REC == REC_WENO5Z) && !P::sr;
   d.sweep[0] = k_sweep<P, REC, RS, ND, 0, T>;
   d.sweep[1] = k_sweep<P, REC, RS, ND, 1, T>;
   if constexpr (ND == 3) d.sweep[2] = k_sweep<P, REC, RS, ND, 2, T>;

@@ -287,9 +287,8 @@ program amun_host
                                    ": ", trim(amun_dev_last_error())
     stop 2
   end if
-  ! one launch per stage (bitwise the per-direction launches' results) where
-  ! the library builds it; the configurations it does not cover return 600
-  ! and keep the per-direction launches
+  ! times per stage instead of per sweep in amun_dev_timed_run; the launches
+  ! and results are the same, and so is a run whose configuration returns 600
   str = get_str("stage_fusion", "on")
   if (trim(str) == "on" .or. trim(str) == "yes" .or. trim(str) == "true") then
     iret = amun_dev_set_stage_fusion(ctx, 1)

@@ -1,12 +1,12 @@
-"""One launch per stage (amun_dev_set_stage_fusion): the x, y (and z) sweeps
-of a stage run in one kernel whose workgroups hold whole blocks.  Every
-update of a cell reads only its own block's increment, so the fused stage
-must give the per-direction launches' states and time steps bit for bit:
-2D and 3D, HD and MHD, adiabatic and isothermal, TVD and WENO5-Z, FP64 and
-mixed, with viscous, resistive and gravity sources, multi-level meshes,
-batches of grids and captured graphs.  The reference has one update_fluxes
-per stage (evolution.F90:628-1208); the split launches are pinned to the
-oracle elsewhere, so equality here carries that parity over."""
+"""Launch shapes and the stage switch (amun_dev_set_stage_fusion).
+
+The configurations of CASES (2D and 3D, HD and MHD, adiabatic and isothermal,
+TVD and WENO5-Z, Roe, blocks of 4 to 16 cells, viscous, resistive and gravity
+sources) take one step against the oracle, and several with every workgroup
+size and order of amun_dev_set_launch, which must give the same bits: the
+workgroups, and so the pencils and tiles of a lane, differ, the arithmetic of
+a cell does not.  The stage switch changes the times that amun_dev_timed_run
+reports and nothing else; on, off and toggled, the results are the same."""
 import os
 import sys
 
@@ -15,11 +15,13 @@ import pytest
 
 from amun_amd.config import Params, c1_params, c2_params
 from amun_amd.problems import cell_centres, initial_state, prim_to_cons
-from amun_amd.solver import AmrSolver, AmunError, Batch, Solver
+from amun_amd.solver import AmunError, Solver
 
 GOLD = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden")
 sys.path.insert(0, GOLD)
 from make_golden import grav_params, grav_state  # noqa: E402
+import oracle_lib as ol  # noqa: E402
+from test_gpu_parity import relerr  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
@@ -66,102 +68,90 @@ CASES = {
 }
 
 
-def _run(p, u0, nsteps, fused, graph=False):
+def _case(name):
+    p = CASES[name]()
+    if name.startswith("grav"):
+        return p, grav_state(p)
+    return p, initial_state(p) if name.startswith("c") else noisy(p, 17)
+
+
+@pytest.mark.parametrize("name", [n for n in CASES if CASES[n]().precision == "fp64"])
+def test_one_step_vs_oracle(name):
+    p, u0 = _case(name)
+    print(f"[case] one step {name}", flush=True)
+    o = ol.OracleRun(p)
+    o.set_state(u0)
+    tr = o.run(1)
     with Solver(p) as s:
-        s.set_graph(graph)
-        if fused:
-            s.set_stage_fusion(True)
         s.upload(u0)
-        dts = s.run(nsteps)
-        return s.download(), dts, s.statistics()
+        dt, _ = s.advance()
+        ug = s.download()
+    assert dt == pytest.approx(tr[0, 0], rel=1e-13)
+    assert relerr(ug, o.get_state()).max() <= 1e-12
+
+
+def _shapes(nd):
+    sizes = (64, 128, 256) if nd == 3 else (256,)
+    return [[(256, z)] * 2 + [(wg, z)] * (nd - 2) for wg in sizes for z in (0, 1)]
 
 
 @pytest.mark.parametrize("name", list(CASES))
-def test_fused_equals_split(name):
-    p = CASES[name]()
-    u0 = initial_state(p) if name.startswith("c") else noisy(p, 17)
-    if name.startswith("grav"):
-        u0 = grav_state(p)
-    print(f"[case] fusion {name}", flush=True)
-    us, ds, ss = _run(p, u0, 5, False)
-    uf, df, sf = _run(p, u0, 5, True)
-    np.testing.assert_array_equal(df, ds)
-    np.testing.assert_array_equal(uf, us)
-    np.testing.assert_array_equal(sf, ss)
+def test_launch_shapes_agree(name):
+    """Five steps in every launch shape: states, time steps and statistics
+    bit for bit those of the default."""
+    p, u0 = _case(name)
+    print(f"[case] shapes {name}", flush=True)
+    with Solver(p) as s:
+        want = None
+        for shape in [None] + _shapes(p.ndims):
+            if shape:
+                s.set_launch(shape)
+            s.upload(u0)
+            got = s.run(5), s.download(), s.statistics()
+            want = want or got
+            for a, b in zip(got, want):
+                np.testing.assert_array_equal(a, b)
 
 
-def test_fused_graph_replays_and_toggle():
-    """Captured graphs of the fused step replay to the eager results, and
-    switching the fusion off and on between steps keeps the run exact."""
+@pytest.mark.parametrize("graph", [False, True])
+def test_stage_switch_changes_no_result(graph):
+    """On, off and toggled between the steps, launched and replayed."""
     p = c2_params(32)
     u0 = initial_state(p)
-    print("[case] fusion graphs and toggling", flush=True)
-    us, ds, _ = _run(p, u0, 6, False)
-    ug, dg, _ = _run(p, u0, 6, True, graph=True)
-    np.testing.assert_array_equal(dg, ds)
-    np.testing.assert_array_equal(ug, us)
+    print(f"[case] stage switch graph={graph}", flush=True)
     with Solver(p) as s:
         s.upload(u0)
-        dts = []
-        for k in range(6):
-            s.set_stage_fusion(k % 2 == 0)
-            dts.append(s.run(1)[0])
-        np.testing.assert_array_equal(np.asarray(dts), ds)
-        np.testing.assert_array_equal(s.download(), us)
+        want = s.run(6), s.download()
+    for on in (lambda k: True, lambda k: k % 2 == 0):
+        with Solver(p) as s:
+            s.set_graph(graph)
+            s.upload(u0)
+            dts = []
+            for k in range(6):
+                s.set_stage_fusion(on(k))
+                dts.append(s.run(1)[0])
+            np.testing.assert_array_equal(dts, want[0])
+            np.testing.assert_array_equal(s.download(), want[1])
 
 
-def test_fused_per_kernel_timing():
-    """One timed event per stage with the fusion on (SSPRK(3,3): 3 stages
-    and the end-of-step kernel)."""
+def test_times_per_stage():
+    """Three stages and the end of the step with the switch on, nine sweeps
+    and the end with it off; the tuner needs the sweeps' own times."""
     with Solver(c2_params(32)) as s:
         s.upload(initial_state(c2_params(32)))
         s.set_stage_fusion(True)
         ms, kms = s.timed_run(2, per_kernel=True)
-        print(f"[case] fused timing {ms:.3f} ms, {kms}", flush=True)
+        print(f"[case] stage times {ms:.3f} ms, {kms}", flush=True)
         assert len(kms) == 4 and all(k > 0 for k in kms)
         with pytest.raises(AmunError, match="fused stage off"):
             s.autotune(1)
-
-
-@pytest.mark.parametrize("nd", [2, 3])
-def test_fused_amr_equals_split(nd):
-    from test_gpu_amr import _case
-    p, meta, u0 = _case(nd, rec="weno5z" if nd == 3 else "tvd")
-    print(f"[case] fusion AMR {nd}D blocks={len(meta)}", flush=True)
-    out = []
-    for fused in (False, True):
-        with AmrSolver(p, meta) as s:
-            if fused:
-                s.set_stage_fusion(True)
-            s.upload(u0)
-            dts = s.run(4)
-            out.append((s.download(), dts))
-    np.testing.assert_array_equal(out[1][1], out[0][1])
-    np.testing.assert_array_equal(out[1][0], out[0][0])
-
-
-def test_fused_batch_equals_split():
-    from test_gpu_batch import _kh_runs
-    from amun_amd.problems import kelvin_helmholtz_2d
-    common, runs = _kh_runs([64, 32, 96])
-    u0s = [kelvin_helmholtz_2d(p, seed=60 + i) for i, p in enumerate(runs)]
-    print("[case] fusion batch", flush=True)
-    out = []
-    for fused in (False, True):
-        with Batch(common, runs) as b:
-            if fused:
-                b.set_stage_fusion(True)
-            for r, u0 in enumerate(u0s):
-                b.upload(r, u0)
-            dts = b.run(5)
-            out.append(([b.download(r) for r in range(len(runs))], dts))
-    np.testing.assert_array_equal(out[1][1], out[0][1])
-    for a, b in zip(out[1][0], out[0][0]):
-        np.testing.assert_array_equal(a, b)
+        s.set_stage_fusion(False)
+        ms, kms = s.timed_run(2, per_kernel=True)
+        assert len(kms) == 10 and all(k > 0 for k in kms)
 
 
 @pytest.mark.parametrize("cfg", ["crmp5", "srmhd", "ncells12"])
-def test_fusion_refused_where_not_built(cfg):
+def test_stage_switch_refused(cfg):
     if cfg == "crmp5":
         p = _cfg(2, "hd", "crmp5", "hllc", n=16)
         p.nghosts = 4
