@@ -92,23 +92,20 @@ def cpu_baseline(p_full):
                                    f"{n1} steps, FP64, {secs1:.2f} s on one host thread"}}
 
 
-def c3_legs(steps: int, warmup: int, launch: str):
+def c3_legs(steps: int, warmup: int):
     """The batched/AMR configuration beside the headline: the 64-grid KH
     batch (one block pool, per-run dt) and the 3-level 3D AMR mesh of 6224
     leaves of 16^3, FP64 and mixed, and the 2D HD 128^2 grid (launch-bound),
     steps replayed from captured graphs; zone-updates/s over all interior
-    cells.  Each is timed with one launch per sweep direction and with one
-    launch per stage; `value` and `ms_per_step` follow `launch`."""
+    cells."""
     from amun_amd.config import c1_params, c3_batch_params
     from amun_amd import mesh
     from amun_amd.problems import initial_state, kelvin_helmholtz_2d
     from amun_amd.solver import AmrSolver, Batch, Solver
 
-    def timed(make, upload, fused, nsteps):
+    def timed(make, upload, nsteps):
         with make() as s:
             upload(s)
-            if fused:
-                s.set_stage_fusion(True)
             s.set_graph(True)
             s.run(warmup)
             s.sync()
@@ -118,12 +115,9 @@ def c3_legs(steps: int, warmup: int, launch: str):
             return time.perf_counter() - t0, s.info() if hasattr(s, "info") else {}
 
     def leg(make, upload, cells, nsteps=steps, **extra):
-        ws, info = timed(make, upload, False, nsteps)
-        wf, _ = timed(make, upload, True, nsteps)
-        w = wf if launch == "fused" else ws
+        w, info = timed(make, upload, nsteps)
         return {"value": cells * nsteps / w, "unit": "zone-updates/s",
-                "ms_per_step": w / nsteps * 1e3, "ms_per_step_split": ws / nsteps * 1e3,
-                "ms_per_step_fused": wf / nsteps * 1e3, "cells": cells, **extra}, info
+                "ms_per_step": w / nsteps * 1e3, "cells": cells, **extra}, info
 
     def upload_batch(runs):
         def up(b):
@@ -165,12 +159,12 @@ def main():
     ap.add_argument("--precision", default="fp64", choices=["fp64", "mixed"])
     ap.add_argument("--no-mixed", action="store_true",
                     help="skip the mixed-precision leg reported beside the FP64 value")
-    ap.add_argument("--launch", default="fused", choices=["fused", "split"],
-                    help="with amun_dev_set_stage_fusion (timings per stage) or without "
-                         "(timings per sweep); the launches are the same; the other is "
-                         "reported beside the value")
+    ap.add_argument("--launch", default="split", choices=["fused", "split"],
+                    help="kernel_ms_per_step of every stage (fused, "
+                         "amun_dev_set_stage_fusion) or every sweep (split); the launches "
+                         "are the same")
     ap.add_argument("--no-other-launch", action="store_true",
-                    help="skip the FP64 leg of the other launch mode")
+                    help="no effect: one leg times the launches")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--no-c3", action="store_true",
                     help="skip the batched/AMR legs (64 KH grids, 6224-leaf AMR mesh)")
@@ -212,13 +206,12 @@ def main():
     print(f"[bench] building {args.size}^3 initial state", file=sys.stderr, flush=True)
     u0 = initial_state(p)
 
-    def measure(params, launch):
-        fused = launch == "fused"
+    def measure(params):
         s = Solver(params)
-        if fused:
+        if args.launch == "fused":
             s.set_stage_fusion(True)
         s.upload(u0)
-        tag = params.precision + (" fused" if fused else "")
+        tag = params.precision
         print(f"[bench] {tag}: warmup {args.warmup} steps", file=sys.stderr, flush=True)
         s.run(args.warmup)
         s.sync()
@@ -235,20 +228,11 @@ def main():
         s.close()
         return wall, dev_ms, kms
 
-    wall, dev_ms, kms = measure(p, args.launch)
-    # the same step in the other launch mode (bitwise the same results)
-    other_name = "split" if args.launch == "fused" else "fused"
-    other = None
-    if not args.no_other_launch:
-        wo, do, ko = measure(p, other_name)
-        other = {"value": cells * args.steps / wo, "ms_per_step": wo / args.steps * 1e3,
-                 "device_ms_per_step": do / args.steps,
-                 f"speedup_of_{args.launch}": wo / wall,
-                 "kernel_ms_per_step": [round(float(x), 4) for x in ko]}
+    wall, dev_ms, kms = measure(p)
     mixed = None
     if args.precision == "fp64" and not args.no_mixed:
         pm = c2_params(args.size, precision="mixed")
-        wm, dm, km = measure(pm, args.launch)
+        wm, dm, km = measure(pm)
         mixed = {"value": cells * args.steps / wm, "ms_per_step": wm / args.steps * 1e3,
                  "speedup_vs_fp64": wall / wm,
                  "roofline_frac": bytes_per_zone_update(pm) * cells / (dm / args.steps * 1e-3)
@@ -261,8 +245,7 @@ def main():
     achieved = bpz * cells / (step_ms * 1e-3) / 1e9
     traffic = None
     valu = None
-    tf = os.path.join(ROOT, "profiles",
-                      f"traffic_c2_{args.size}_{args.precision}_{args.launch}.json")
+    tf = os.path.join(ROOT, "profiles", f"traffic_c2_{args.size}_{args.precision}.json")
     if os.path.exists(tf):
         prof = json.load(open(tf))
         traffic = prof.get("hbm_bytes_per_step")
@@ -301,17 +284,15 @@ def main():
         "data": "synthetic (seeded random-phase Fourier v and B, rho=1, p=0.6)",
         "config": {"workload": f"3D MHD-GLM WENO5-Z+HLLD SSPRK(3,3) {args.size}^3 "
                                f"as {p.nblocks} blocks of 16^3, CFL 0.3, periodic",
-                   "precision": args.precision, "launch": args.launch, "cells": cells},
+                   "precision": args.precision, "cells": cells},
         "roofline": roofline,
     }
     if valu is not None:
         out["valu"] = valu
-    if other is not None:
-        out[other_name] = other
     if mixed is not None:
         out["mixed"] = mixed
     if not args.no_c3:
-        out["c3"] = c3_legs(args.steps, args.warmup, args.launch)
+        out["c3"] = c3_legs(args.steps, args.warmup)
     if not args.no_cpu_baseline:
         print("[bench] CPU baseline", file=sys.stderr, flush=True)
         out["cpu_baseline"] = cpu_baseline(p)
