@@ -1,8 +1,7 @@
 """The allocation-free cons2prim entry point (amun_dev_cons2prim_noalloc)
 against amun_dev_unit_cons2prim, through the C-ABI: relativistic states with
-failing recoveries (the event counters live in the library's static device
-array), two calls in a row, the second on fewer states, bit for bit; and an
-HD call on the same counters afterwards."""
+failing recoveries (counted in the caller's device array), two calls in a row,
+the second on fewer states, bit for bit; and an HD call afterwards."""
 import ctypes
 import os
 
