@@ -243,7 +243,7 @@ __device__ __forceinline__ void riemann(const EosConst<T>& e, const SrConst& sc,
   else riemann_hll<P, T>(e, cmax, cmax2, ql, qr, f);
 }
 
-// lanes of the x and y sweeps' workgroups
+// the most lanes of a sweep's workgroup (launch.h)
 constexpr int kSweepLanes = 256;
 
 // maximum speed of one sweep workgroup for the next CFL step, and its run
@@ -1514,7 +1514,7 @@ __device__ __forceinline__ double sweep_cells(const SweepArgs& a, const RunConst
 
 // One sweep: the workgroup's pencils are np consecutive ones of the pool.
 template <class P, int REC, int RS, int ND, int DIR, typename T>
-__global__ __launch_bounds__(512, (sweep_min_waves<P, RS, T>()))
+__global__ __launch_bounds__(kSweepLanes, (sweep_min_waves<P, RS, T>()))
 void k_sweep(SweepArgs a, RunConst rc) {
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr bool kLast = DIR == ND - 1;

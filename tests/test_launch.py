@@ -47,7 +47,7 @@ def shapes(tmp_path_factory):
 def test_shapes_cover_every_pencil(shapes):
     for nd, nv, es, sr, R, d, nc, wg, np_, lanes, grid, lds, _ in shapes:
         total = 37 * nc ** (nd - 1)
-        assert np_ % 2 == 0 and np_ * (nc + 2) <= lanes <= max(wg, (2 * (nc + 2) + 63) // 64 * 64) <= 512
+        assert np_ % 2 == 0 and np_ * (nc + 2) <= lanes <= max(wg, (2 * (nc + 2) + 63) // 64 * 64) <= 256
         assert (grid - 1) * np_ < total <= grid * np_
 
 
