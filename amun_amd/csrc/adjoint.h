@@ -250,11 +250,14 @@ __global__ __launch_bounds__(256) void k_tlm_face(const double* __restrict__ X, 
 // lF, GF(i) = (dF/dgamma) . lF.
 // A workgroup takes 64 faces: its waves form the face states and lF variable
 // by variable in LDS, then evaluate the Jacobian column by column (of
-// blockIdx.y's share of them), each lane one face and one column (Dual<1>: about twice the solver's registers, two
-// waves per SIMD).  Bound by VALU issue.  One lane per face with four columns
-// at a time spilled 2 KB a lane and gave a 128^2 grid a quarter of the
-// chip's SIMDs: 595 us (x) and 637 us (y) a launch at 128^2 MHD HLLD, now
-// 54 and 49.
+// blockIdx.y's share of them), each lane one face and one column (Dual<1>:
+// about twice the solver's registers, two waves per SIMD).  Bound by VALU issue
+// where that holds in 256 registers (HD; MHD HLL and, with 30 spilled, HLLC);
+// MHD HLLD spills 106 of them (372 to 380 B a lane) and MHD Roe 416 to 424 (2.7
+// KB), which they wait for besides.  One lane per face with four columns at a
+// time spilled 2 KB a lane with HLLD and gave a 128^2 grid a quarter of the
+// chip's SIMDs: 595 us (x) and 637 us (y) a launch at 128^2 MHD HLLD, now 54
+// and 49.
 constexpr int kAdjFaces = 64;
 template <class P, int RS, int ND, int DIR, typename TF>
 __global__ __launch_bounds__(256, 2) void k_adj_face(

@@ -130,11 +130,11 @@ __device__ __forceinline__ double dt_of(const RunConst& rc, const RunState* R,
 
 // Position of cell (i,j,k) inside a block's variable plane.  Cells are stored
 // in 4x4 x-y bricks: one 128-byte line holds x = 4i'..4i'+3 of four
-// consecutive y, so the x, y and z sweeps (lanes across the two transverse
-// directions, walking the third) each touch few lines per load and reuse
-// them within four steps.  Requires nc % 4 == 0.
-// FP32 arrays (element size 4) of 3D runs use 4x4x2 bricks instead, so that
-// a line (32 floats) again spans four steps of every sweep direction.
+// consecutive y.  Four pencils side by side and four cells of each (x, y), or
+// sixteen pencils (z), are whole lines, and the lanes of a sweep go over them
+// in that order.  Requires nc % 4 == 0.
+// FP32 arrays (element size 4) of 3D runs use 4x4x2 bricks instead: a line (32
+// floats) is again four cells along x and y, of two z planes.
 // All factors are below 2^24, which the masks tell the compiler: the products
 // are the full-rate 24-bit ones (a 32-bit product takes four times as long).
 __host__ __device__ __forceinline__ int mul24(int a, int b) {
@@ -1088,10 +1088,18 @@ __device__ __forceinline__ void reset_speed(const SweepArgs& a, const RunConst& 
 #include "mlp.h"
 
 // Waves per SIMD the sweeps are compiled for.  One lane works on one cell, so
-// that besides the HLLD temporaries (118 registers in FP64) nothing has to
-// stay in registers over a solve: four waves per SIMD (128 registers) hide
-// the FP64 latencies.  The relativistic solvers (quartic, root search) and
-// the Roe eigensystem need more registers.
+// that besides the HLLD temporaries (114 to 121 registers in FP64 MHD with
+// WENO5-Z, 104 to 120 with TVD) nothing has to stay in registers over a solve:
+// four waves per SIMD (128 registers) hide the FP64 latencies.  The
+// relativistic solvers (quartic, root search) and the Roe eigensystem need
+// more registers.
+// In FP64 MHD the reconstructions that keep more of a window alive spill at
+// 128: MP7 180 to 188 B a lane, PPM 68 to 104, GP 52 to 60, MP5 28 to 40, MGP
+// 28 to 40.  Measured, us of a 96^3 HLLD step in blocks of 16 (of 8 in
+// brackets) at four, three and two waves: WENO5-Z 664, 660, 654 (731, 726,
+// 726); MP5 987, 989, 989 (1076, 1087, 1081); PPM 1140, 1106, 1113 (1312,
+// 1252, 1256); GP 1072, 1002, 1001 (1190, 1096, 1092); MP7 1330, 1026, 1089
+// (1514, 1133, 1200); MGP 36.7, 38.8, 35.8 ms.
 template <class P, int RS, typename T>
 constexpr int sweep_min_waves() {
   if (P::sr) return P::mhd ? 2 : 3;
@@ -1115,12 +1123,11 @@ __device__ __forceinline__ X& at_byte(X* x, unsigned o) {
   return *reinterpret_cast<X*>(reinterpret_cast<B*>(x) + o);
 }
 
-// The sweep along DIR of the pencils g0 .. g0 + np - 1 of the pool (np
-// even), one lane per cell.  The cells are
-// staged in LDS; each lane reconstructs its cell, leaves its upper face state
-// in LDS, solves the Riemann problem of its lower face with the state of the
-// cell before it, leaves the flux in LDS and updates its cell with the flux of
-// the cell behind it.  The interior lanes go over the cells in the order of
+// The sweep along DIR of the pencils g0 .. g0 + np - 1 of the pool (np even),
+// one lane per cell.  The cells are staged in LDS; each lane reconstructs its
+// cell, leaves its upper face state in LDS, solves the Riemann problem of its
+// lower face with the state of the cell before it, leaves the flux in LDS and
+// updates its cell with the flux of the cell behind it.  The interior lanes go over the cells in the order of
 // the 4-cell bricks, so that every access of a wave to its own cells is whole
 // 128-byte lines: with a pencil's cells on consecutive lanes instead, the z
 // sweep of the 128^3 MHD run sent 14.2 M write requests to L2 for 4.7 M full
@@ -1130,13 +1137,16 @@ __device__ __forceinline__ X& at_byte(X* x, unsigned o) {
 // (kEarly: the states and the increment too, which a solver of 40 bytes a cell
 // leaves registers for; where it does not, the increment waits in LDS).
 // 256^3 MHD WENO5-Z + HLLD: FP64 11.55 -> 11.07 ms a step, mixed 8.08 -> 7.56.
-// What bounds it: x and y vector issue and latency (0.99 and 1.0 ms a launch
+// What bounds it: x and y vector issue and latency (1.01 and 1.04 ms a launch
 // at 256^3 in FP64; 1.29 and 1.59 with a pencil a lane), z the bytes of the
-// state, its stages and the increment (1.75 ms, 4.2 TB/s, where a device copy
+// state, its stages and the increment (1.72 ms, 4.7 TB/s, where a device copy
 // reaches 5.0).  With a pencil a lane a grid of few cells left most SIMDs idle:
 // 128^2 HD TVD 281 -> 40 us a step, 340^2 MHD 707 -> 98, 512^2 SRMHD stages
-// 1168 -> 224.  Every thread of the workgroup must call this.  Returns the maximum speed of the lane's new state (last sweep of a
-// step).
+// 1168 -> 224.  Blocks of 8 cells take more LDS (FP64 MHD WENO5-Z along y 55 KB
+// a workgroup, two a CU, against 40 KB and four at 16), and a 96^3 step 731 us
+// against 664.
+// Every thread of the workgroup must call this.  Returns the maximum speed of
+// the lane's new state (last sweep of a step).
 template <class P, int REC, int RS, int ND, int DIR, typename T>
 __device__ __forceinline__ double sweep_cells(const SweepArgs& a, const RunConst& rc, int g0,
                                               int np, T* smem, int& run) {

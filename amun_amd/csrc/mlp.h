@@ -13,7 +13,7 @@
 // The process reads all directions, so k_mlp evaluates the slopes dq(d)
 // beforehand from the stage input: for every interior cell of every real
 // block (S) and, block by block, for the cells just beyond each face that
-// a pencil walk reconstructs (G: the cell before the first and after the
+// a sweep reconstructs (G: the cell before the first and after the
 // last of every pencil, through the block's own neighbour table, so that
 // neighbour, virtual and ghost blocks all serve).  The sweeps then only
 // compare and reset (mlp_apply).

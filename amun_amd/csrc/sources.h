@@ -10,7 +10,7 @@
 // 0.5 (u(i+1) - u(i-1)) / dh (operators.F90:181-308), summed over the
 // directions in order, at the cell size of the block's level.  The terms
 // read the stage input's primitive state one cell around each cell in every
-// direction, which the pencil walks of the sweeps do not hold, so a kernel
+// direction, which a sweep stages along its own only, so a kernel
 // computes the eight products per cell beforehand and the last sweep of the
 // stage subtracts them from the completed increment in the reference's
 // order (k_sweep).  Products and differences are rounded as the reference
