@@ -2,7 +2,8 @@
 go wrong: blocks of 4 to 64 cells (odd numbers of 4-cell rows, pencils that do
 not fill a workgroup, workgroups over several blocks), launches on both sides
 of the small-grid rule, adjoint faces over several tiles, fine faces of small
-blocks, a handful of states, and downloads on both sides of the staged copy."""
+blocks, a handful of states, and transfers on both sides of the rules that
+convert them on the host, in one piece or through staged ones."""
 import ctypes
 
 import numpy as np
