@@ -12,6 +12,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <new>
 #include <thread>
 
 // ===========================================================================
@@ -1205,14 +1206,16 @@ static int pool_to_grid(amun_ctx* c, int r, const void* X, size_t es, double* u)
   const dim3 grid(transfer_grid(n).x, c->nv);
   Transfer t(c);
   HIP_TRY(t.err);
-  if (bytes <= kHostBytes) {
-    std::vector<double> h(bytes / sizeof(double));
+  // without host memory for it, the larger ones' way
+  std::unique_ptr<double[]> h;
+  if (bytes <= kHostBytes) h.reset(new (std::nothrow) double[bytes / sizeof(double)]);
+  if (h) {
     const GridShape s = run_shape(c, r);
     HIP_TRY(hipStreamSynchronize(c->stream));
-    HIP_TRY(hipMemcpy(h.data(), static_cast<const char*>(X) + s.b0 * per * es,
+    HIP_TRY(hipMemcpy(h.get(), static_cast<const char*>(X) + s.b0 * per * es,
                       bytes / sizeof(double) * es, hipMemcpyDeviceToHost));
-    if (es == sizeof(double)) blocks_to_grid(s, c->rc, c->nv, h.data(), u);
-    else blocks_to_grid(s, c->rc, c->nv, reinterpret_cast<const float*>(h.data()), u);
+    if (es == sizeof(double)) blocks_to_grid(s, c->rc, c->nv, h.get(), u);
+    else blocks_to_grid(s, c->rc, c->nv, reinterpret_cast<const float*>(h.get()), u);
     return 0;
   }
   if (es == sizeof(double))
@@ -1269,16 +1272,16 @@ static int blocks_to_pool(amun_ctx* c, const double* u, int m, int ng) {
 // with the gather and without: one 32^2 block 30, 42; 8^3 blocks of two ghost
 // layers 2.3 MB 159, 313; 18 MB 1449, 2176; 4.6 MB of 8^2 274, 377; of 32^2
 // 275, 236; 18 MB of 16^3 1383, 1131; larger arrays come from fresh pages at
-// 4 GB/s).  h holds the gathered
-// rows, which the stream reads until it is waited for.
+// 4 GB/s).  h holds the gathered rows, which the stream reads until it is
+// waited for.
 static int ghosted_to_pool(amun_ctx* c, const double* u, std::unique_ptr<double[]>& h) {
   const int ng = c->cfg.nghosts, m = c->rc.nc + 2 * ng;
   const size_t n = c->rc.nblk * (size_t)c->nv * c->rc.ncell, inner = n * sizeof(double);
   const size_t full = inner / c->rc.ncell * m * m * (c->rc.nd == 3 ? m : 1);
-  if (!(inner <= (1u << 20) || (inner <= (8u << 20) && 2 * full > 3 * inner) ||
-        (inner <= (24u << 20) && full > 3 * inner)))
-    return blocks_to_pool(c, u, m, ng);
-  h.reset(new double[n]);
+  if (inner <= (1u << 20) || (inner <= (8u << 20) && 2 * full > 3 * inner) ||
+      (inner <= (24u << 20) && full > 3 * inner))
+    h.reset(new (std::nothrow) double[n]);
+  if (!h) return blocks_to_pool(c, u, m, ng);
   interiors_of(c->rc, c->nv, ng, c->rc.nblk, u, h.get());
   return blocks_to_pool(c, h.get(), c->rc.nc, 0);
 }
@@ -1311,30 +1314,35 @@ static int download_blocks_virtual(amun_ctx* c, double* u, double* q) {
     return hipGetLastError();
   };
   // Arrays that U1 does not hold go through it in pieces, each of which waits
-  // for the one before.  Small ones take an allocation instead, and the
-  // smallest one copy for both (us a download of u and q: 28 blocks of 8^2
-  // MHD of three levels 200 in pieces, 111 with an allocation; four of 16^2
-  // HD with open sides 101, 58, and 41 with one copy).
+  // for the one before.  Small ones take an allocation, if there is one to be
+  // had, and the smallest one copy for both (us a download of u and q: 28
+  // blocks of 8^2 MHD of three levels 200 in pieces, 111 with an allocation;
+  // four of 16^2 HD with open sides 101, 58, and 38 with one copy).
   const size_t n = rc.nblk * per, bytes = n * sizeof(double);
   if (bytes <= kWholeBytes) {
     Transfer t(c);
     HIP_TRY(t.err);
     double* buf = nullptr;
-    HIP_TRY(hipMalloc((void**)&buf, (q ? 2 : 1) * bytes));
-    hipError_t e = pack(c->U0, buf, 0, rc.nblk);
-    if (e == hipSuccess && q) e = pack(nullptr, buf + n, 0, rc.nblk);
-    if (e == hipSuccess && q && bytes <= kPairBytes) {
-      std::unique_ptr<double[]> h(new double[2 * n]);
-      e = hipMemcpyAsync(h.get(), buf, 2 * bytes, hipMemcpyDeviceToHost, c->stream);
-      if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-      std::memcpy(u, h.get(), bytes);
-      std::memcpy(q, h.get() + n, bytes);
-    } else if (e == hipSuccess) {
-      r = copy_to_host(c, u, buf, bytes);
-      if (!r && q) r = copy_to_host(c, q, buf + n, bytes);
+    if (hipMalloc((void**)&buf, (q ? 2 : 1) * bytes) == hipSuccess) {
+      hipError_t e = pack(c->U0, buf, 0, rc.nblk);
+      if (e == hipSuccess && q) e = pack(nullptr, buf + n, 0, rc.nblk);
+      std::unique_ptr<double[]> h;
+      if (q && bytes <= kPairBytes) h.reset(new (std::nothrow) double[2 * n]);
+      if (e == hipSuccess && h) {
+        e = hipMemcpyAsync(h.get(), buf, 2 * bytes, hipMemcpyDeviceToHost, c->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+        if (e == hipSuccess) {
+          std::memcpy(u, h.get(), bytes);
+          std::memcpy(q, h.get() + n, bytes);
+        }
+      } else if (e == hipSuccess) {
+        r = copy_to_host(c, u, buf, bytes);
+        if (!r && q) r = copy_to_host(c, q, buf + n, bytes);
+      }
+      (void)hipFree(buf);
+      return e == hipSuccess ? r : fail(1000 + (int)e, "download_blocks");
     }
-    (void)hipFree(buf);
-    return e == hipSuccess ? r : fail(1000 + (int)e, "download_blocks");
+    (void)hipGetLastError();
   }
   for (int pass = 0; pass < 2 && !r; pass++) {
     double* dst = pass == 0 ? u : q;
